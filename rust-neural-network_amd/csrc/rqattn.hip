@@ -582,16 +582,16 @@ static void attn_splits(int64_t wgs, int64_t T, bool wide, int64_t &ns, int64_t 
     ns = T > 0 ? ceil_div(T, tps) : 1;  // no empty split
 }
 
-// Split workspace: a count per query and range (the first bytes, rounded up
-// to 256), then the splits' states [query][split][2 + 3 ng].
-static size_t attn_count_bytes(int64_t queries) {
-    return (size_t)ceil_div(4 * queries, 256) * 256;
+// Split workspace: the counts (one per query and range), then the splits'
+// states [query][split][2 + 3 ng]. The counts' area is the same for every
+// shape -- a call splits only while its workgroups number fewer than
+// kWideWgsPerCu per CU (attn_splits) -- so a workspace left by one shape holds
+// zeros where another shape's counts are.
+static size_t attn_count_bytes() {
+    return (size_t)ceil_div(4 * (int64_t)kWideWgsPerCu * device_cu_count(), 256) * 256;
 }
 static size_t attn_split_bytes(int64_t queries, int64_t ns, int64_t ng) {
-    const int64_t ranges = ng > 64 ? ceil_div(ng, kWideRange) : 1;  // a count per range
-    return ns > 1 ? attn_count_bytes(queries * ranges) +
-                        (size_t)(queries * ns * (2 + 3 * ng)) * sizeof(float)
-                  : 0;
+    return ns > 1 ? attn_count_bytes() + (size_t)(queries * ns * (2 + 3 * ng)) * sizeof(float) : 0;
 }
 
 static size_t attn_workspace_bytes(int64_t bh, int64_t nq, int64_t seq, int64_t dim) {
@@ -716,7 +716,7 @@ extern "C" int rnn_rotorquant_kv_attention_ws(const float *q, int64_t bh, int64_
     }
     uint32_t *cnt = static_cast<uint32_t *>(ws);
     float *part = ws ? reinterpret_cast<float *>(static_cast<uint8_t *>(ws) +
-                                                 attn_count_bytes(bh * nq * nranges))
+                                                 attn_count_bytes())
                      : nullptr;
     if (ng > 64) {
         rq_kv_attn_wide_kernel<<<dim3(grid, (unsigned)nranges, (unsigned)ns), kAttnWaves * 64,

@@ -157,3 +157,31 @@ def test_kv_attention_split_workspace_and_alloc(dev, hip):
     with pytest.raises(hip.RnnError, match="workspace"):
         hip.rotorquant_kv_attention(q, kp, vp, krot, vrot, seq, 0.125, workspace=ws[: need - 4])
     assert hip.rotorquant_kv_attention_workspace_size(1024, 1, seq, dim) == 0  # queries fill it
+
+
+def test_kv_attention_workspace_shared_between_shapes(dev, hip):
+    """The counts of every shape lie in one area of the workspace: a call with
+    more queries after one with fewer (whose states would otherwise lie where
+    the second's counts are), and the reverse, on the wrapper's cached
+    workspace, each equal to the call with a fresh workspace bit for bit."""
+    import torch
+    dim, seq = 64, 1100
+    ng = (dim + 2) // 3
+    rot = to_dev(W.rotors(ng, seed=31), dev)
+    runs = []
+    for bh, nq in ((2, 1), (24, 4), (3, 1)):
+        kp, _ = make_cache(hip, dev, W.activations(bh * seq, dim, seed=bh), W.rotors(ng, seed=31),
+                           4, bh, seq, hip.RQ_PAGE_K)
+        vp, _ = make_cache(hip, dev, W.activations(bh * seq, dim, seed=bh + 1),
+                           W.rotors(ng, seed=31), 4, bh, seq, hip.RQ_PAGE_V)
+        q = torch.randn((bh, nq, dim), device=dev)
+        need = hip.rotorquant_kv_attention_workspace_size(bh, nq, seq, dim)
+        assert need > 0
+        runs.append((q, kp, vp, rot, rot, seq, 0.125))
+        fresh = hip.rotorquant_kv_attention(*runs[-1], workspace=torch.zeros(
+            need, dtype=torch.uint8, device=dev))
+        runs[-1] = (runs[-1], fresh)
+    for _ in range(2):
+        for args, fresh in runs:
+            out = torch.full_like(fresh, float("nan"))
+            assert torch.equal(hip.rotorquant_kv_attention(*args, out=out), fresh)
