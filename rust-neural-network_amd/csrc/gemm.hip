@@ -625,6 +625,23 @@ __device__ __forceinline__ void tile_epilogue(const Epilogue &epi, const v4i (&a
     }
 }
 
+// f(std::integral_constant<int, 0>{}), ..., f(std::integral_constant<int, N-1>{}):
+// a loop unrolled by construction, whose body sees its index as a constant.
+template <class Fn, int... Is>
+__device__ __forceinline__ void static_for_impl(Fn &&f, std::integer_sequence<int, Is...>) {
+    (f(std::integral_constant<int, Is>{}), ...);
+}
+template <int N, class Fn>
+__device__ __forceinline__ void static_for(Fn &&f) {
+    static_for_impl(f, std::make_integer_sequence<int, N>{});
+}
+
+}  // namespace rnn
+
+#include "gemm_mid.hpp"
+
+namespace rnn {
+
 // Fragments of one K step held in registers: FM activation blocks, FN weight
 // blocks (16 rows x 64 B each, one 16-byte chunk per lane); for ternary B the
 // lane's 32-bit word of 16 codes (w) is read first and decoded into b.
@@ -894,17 +911,6 @@ void gemm_dma_kernel(const int8_t *__restrict__ A, const int8_t *__restrict__ B,
 //    code whatever the unroller's thresholds.
 constexpr int kL = 128;  // K bytes per stage
 constexpr int kTerLutCopies = 16;  // ternary decode table copies (16 KiB)
-
-// f(std::integral_constant<int, 0>{}), ..., f(std::integral_constant<int, N-1>{}):
-// a loop unrolled by construction, whose body sees its index as a constant.
-template <class Fn, int... Is>
-__device__ __forceinline__ void static_for_impl(Fn &&f, std::integer_sequence<int, Is...>) {
-    (f(std::integral_constant<int, Is>{}), ...);
-}
-template <int N, class Fn>
-__device__ __forceinline__ void static_for(Fn &&f) {
-    static_for_impl(f, std::make_integer_sequence<int, N>{});
-}
 
 __device__ __forceinline__ int swz8(int r) { return (r >> 1) & 7; }
 
@@ -2061,6 +2067,23 @@ static int launch_dma_auto(const int8_t *A, const int8_t *B, int64_t M, int64_t 
     return launch_dma<256, 224, 4, 2, 4>(A, B, M, N, K, epi, st, name);
 }
 
+// K % 16 == 0, 16-byte aligned operands: the prefill kernel where its shape
+// conditions hold and its 256 x 224 tiles fill the CUs, else the small tiles
+// (graph replay, K = 4096: 77 x 4096 16.8 -> 8.7 us, 512 x 4096 37.8 -> 16.4,
+// 512 x 11008 46.8 -> 40.3; K = 2976, N = 257, M = 77 33.4 -> 6).
+static int launch_w8a8_auto(const int8_t *A, const int8_t *B, int64_t M, int64_t N, int64_t K,
+                            const Epilogue &epi, hipStream_t st, const char *name) {
+    const bool pp = dma_ok(A, B, N, K, epi) && l128_fits(M, N, K, false);
+    if (mid_fits(K)) {
+        double cost = 0.0;
+        const MidShape *s = mid_choose<false>(M, N, K, &cost);
+        if (!pp || cost < pp_cost(M, N, K)) return s->run(A, B, M, N, K, epi, st, name);
+    }
+    if (pp) return launch_pp<PrefillCfg>(A, B, M, N, K, epi, st, name);
+    if (dma_ok(A, B, N, K, epi)) return launch_dma_auto(A, B, M, N, K, epi, st, name);
+    return launch_tiled<128, 128, 64, 64, false>(A, B, M, N, K, epi, st, name);
+}
+
 // Decode GEMV dispatch: one-shot workgroups of 4 waves per 16 weight rows,
 // each wave keeping 16 16-byte loads in flight per lane (the whole 4096-wide
 // row block of 64 KiB is requested at once). A persistent variant that walks
@@ -2147,8 +2170,8 @@ extern "C" int rnn_w8a8_linear(const int8_t *aq, const float *sa, const int8_t *
     hipStream_t st = as_stream(stream);
     if (algo == RNN_ALGO_GEMV || (algo == RNN_ALGO_AUTO && m <= 16))
         return launch_gemv(aq, wq, m, n, k, epi, st, name);
-    if (algo == RNN_ALGO_TILED_DMA || (algo == RNN_ALGO_AUTO && dma))
-        return launch_dma_auto(aq, wq, m, n, k, epi, st, name);
+    if (algo == RNN_ALGO_TILED_DMA) return launch_dma_auto(aq, wq, m, n, k, epi, st, name);
+    if (algo == RNN_ALGO_AUTO) return launch_w8a8_auto(aq, wq, m, n, k, epi, st, name);
     return launch_tiled<128, 128, 64, 64, false>(aq, wq, m, n, k, epi, st, name);
 }
 
@@ -2201,6 +2224,16 @@ extern "C" int rnn_ternary_gemm(const int8_t *aq, const float *sa, const uint32_
     // CU. Codes in the reference layout decode through the replicated LDS
     // table; codes in the MFMA layout through byte permutes.
     const bool l128 = k % (kL * L128Ter::KS) == 0 && l128_fits(m, n, k, true);
+    // Codes in the MFMA layout: the small tiles where they are estimated to be
+    // faster, or where the 64 x 128 kernel's conditions (K % 256, N % 4) fail
+    // (graph replay, K = 4096: 4 x 4096 9.6 -> 5.6 us, 16 x 11008 10.1 -> 9.1;
+    // K = 2976, N = 257, M = 4 32.5 -> 5.0, M = 512 41.1 -> 8.6).
+    if (algo == RNN_ALGO_AUTO && mfma_layout && mid_fits(k)) {
+        double cost = 0.0;
+        const MidShape *s = mid_choose<true>(m, n, k, &cost);
+        if (!dma || !l128 || cost < l128_ter_cost(m, n, k))
+            return s->run(aq, pb, m, n, k, epi, st, name);
+    }
     if (algo == RNN_ALGO_TILED_DMA || (algo == RNN_ALGO_AUTO && dma)) {
         if (l128 && mfma_layout) return launch_l128<L128TerPerm>(aq, pb, m, n, k, epi, st, name);
         if (l128) return launch_l128<L128Ter>(aq, pb, m, n, k, epi, st, name);
@@ -2392,10 +2425,7 @@ static int igemm_on_workspace(const uint8_t *a, const int8_t *b, int32_t *c, int
     RNN_TRY(check_launch(name));
     Epilogue epi{nullptr, nullptr, nullptr, nullptr, c, cs, m, n, 0};
     if (m <= 16) return launch_gemv(ap, bt, m, n, kp, epi, st, name);
-    // 64x64 tiles while 128x128 tiles would leave most CUs idle
-    if (ceil_div(m, 128) * ceil_div(n, 128) < cus)
-        return launch_tiled<64, 64, 32, 32, false>(ap, bt, m, n, kp, epi, st, name);
-    return launch_tiled<128, 128, 64, 64, false>(ap, bt, m, n, kp, epi, st, name);
+    return launch_w8a8_auto(ap, bt, m, n, kp, epi, st, name);
 }
 
 // C = 0 for an empty reduction (a fill kernel, safe under graph capture).

@@ -209,6 +209,36 @@ def test_w8a8_small_shapes(dev, hip, m, k, n, algo):
         assert_f32_equal(y, ye)
 
 
+# One shape per tile of the small-tile GEMM that AUTO estimates to be fastest (m x n tile
+# 16x16, 32x16, 32x64, 32x32, 64x64, 48x32, 64x128, 64x32, 128x128, 128x256), ragged in m, n
+# and K, and K of several stages with a partial last one
+SMALL_TILE_SHAPES = [(17, 272, 4), (17, 272, 2049), (17, 272, 8200), (33, 272, 2049),
+                     (33, 272, 8200), (100, 272, 2049), (65, 272, 8200), (250, 272, 1500),
+                     (200, 272, 8200), (2047, 272, 2049), (20, 16, 1), (77, 4112, 300),
+                     (130, 2064, 1001), (64, 4096, 512), (200, 1040, 129)]
+
+
+@pytest.mark.parametrize("m,k,n", SMALL_TILE_SHAPES)
+def test_w8a8_small_tile_gemm(dev, hip, m, k, n):
+    """m > 16 on the small-tile GEMM: int32 and fp32 bit-exact, nothing written
+    past the outputs, outputs at an odd address (the scalar stores), bias + ReLU."""
+    import torch
+    g = W.rng(m + k + n)
+    aq, wq = (g.integers(-128, 128, s).astype(np.int8) for s in ((m, k), (n, k)))
+    sa, sw, bias = (g.random(c).astype(np.float32) - np.float32(0.25) for c in (m, n, n))
+    da, dsa, dw, dsw, db = (to_dev(v, dev) for v in (aq, sa, wq, sw, bias))
+    for b, relu in ((None, False), (bias, True)):
+        ye, acce = O.w8a8_linear(aq, sa, wq, sw, b, relu)
+        for off in (0, 1):
+            y = torch.full((off + m * n + 8,), -3.0, device=dev)
+            acc = torch.full((off + m * n + 8,), -3, dtype=torch.int32, device=dev)
+            hip.w8a8_linear(da, dsa, dw, dsw, None if b is None else db, relu=relu,
+                            y=y[off:off + m * n], acc=acc[off:off + m * n])
+            assert np.array_equal(host(acc[off:off + m * n]).reshape(m, n), acce)
+            assert_f32_equal(host(y[off:off + m * n]).reshape(m, n), ye)
+            assert bool((y[off + m * n:] == -3).all()) and bool((acc[off + m * n:] == -3).all())
+
+
 @pytest.mark.parametrize("m,k,n", [(17, 128, 4), (64, 256, 128), (129, 128, 228), (200, 1024, 300),
                                    (256, 256, 224), (300, 384, 1000), (513, 640, 452),
                                    (1000, 128, 14336 // 16)])

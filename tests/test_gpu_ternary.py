@@ -188,7 +188,13 @@ def test_ternary_prepack_layout(dev, hip):
 
 @pytest.mark.parametrize("m,k,n", [(1, 256, 16), (64, 512, 128), (512, 4096, 512), (37, 48, 29),
                                    (200, 1024, 300), (17, 256, 4), (130, 512, 200),
-                                   (96, 1536, 260), (33, 2048, 132), (64, 768, 128)])
+                                   (96, 1536, 260), (33, 2048, 132), (64, 768, 128),
+                                   # the small-tile GEMM's tiles (m x n): 16x16, 32x16, 32x64,
+                                   # 32x32, 64x64, 48x32, 64x128, 64x32, 128x128, 128x256
+                                   (3, 272, 7), (17, 272, 2049), (17, 272, 8200), (33, 272, 2049),
+                                   (33, 272, 8200), (100, 272, 2049), (65, 272, 8201),
+                                   (250, 272, 1501), (200, 272, 8201), (2047, 272, 2049),
+                                   (5, 4112, 300), (2, 7392, 1001), (130, 1040, 1001)])
 def test_ternary_gemm_mfma_layout(dev, hip, m, k, n):
     """The GEMM on prepacked codes (RNN_FLAG_TERNARY_MFMA_LAYOUT) against the
     oracle on the reference layout: the LDS-DMA kernel (k % 256 == 0; one to
