@@ -281,6 +281,22 @@ int rnn_linear_layer(const float *x, int64_t batch, int64_t in_f,
                      const float *w, int64_t out_f, const float *bias, int relu,
                      float *y, void *stream);
 
+/* rnn_linear_layer (src/tensor.rs:747-800) with scratch: x and W are split
+ * into bf16 parts (x in the workspace, W as it is read) and multiplied on the
+ * bf16 matrix cores, bias and ReLU in the same kernel. `workspace`: 16-byte
+ * aligned, at least rnn_linear_layer_workspace_size(w, batch, in_f, out_f)
+ * bytes, any contents; it depends on the sizes and on the alignment of w, and
+ * is 0 where the call runs as rnn_linear_layer does (few rows or features).
+ * Infinities, NaN and values the parts do not hold are computed in f32.
+ * workspace NULL: as rnn_linear_layer. Calls sharing a workspace must be
+ * ordered on one stream. */
+size_t rnn_linear_layer_workspace_size(const float *w, int64_t batch,
+                                       int64_t in_f, int64_t out_f);
+int rnn_linear_layer_ws(const float *x, int64_t batch, int64_t in_f,
+                        const float *w, int64_t out_f, const float *bias,
+                        int relu, float *y, void *workspace,
+                        size_t workspace_bytes, void *stream);
+
 /* ------------------------------------- QuantizedTensor formats (next row) */
 
 /* QuantFormat (src/quantize.rs:37-56), in the reference's declaration order.

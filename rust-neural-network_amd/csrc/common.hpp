@@ -55,6 +55,13 @@ inline int64_t ceil_div(int64_t a, int64_t b) { return (a + b - 1) / b; }
 // grid-stride kernels (256 CUs on MI355X).
 int device_cu_count();
 
+// sgemm.hip: x . W^T on split operands (x [m, k], W [n, k], contiguous).
+// Scratch bytes it needs, 0 where the f32 kernels are the better ones;
+// `aligned`: k % 4 == 0 and W 16-byte aligned.
+size_t sgemm_nt_scratch(int64_t m, int64_t n, int64_t k, bool aligned);
+int sgemm_nt_split(int64_t m, int64_t n, int64_t k, const float *x, const float *w, const float *bias,
+                   int relu, float *y, void *scratch, hipStream_t st, const char *name);
+
 }  // namespace rnn
 
 #define RNN_REQUIRE(cond, ...)                                          \

@@ -100,16 +100,39 @@ extern "C" int rnn_bias_act(float *y, const float *bias, int64_t rows, int64_t c
     return check_launch(name);
 }
 
-extern "C" int rnn_linear_layer(const float *x, int64_t batch, int64_t in_f, const float *w,
-                                int64_t out_f, const float *bias, int relu, float *y,
-                                void *stream) {
+static bool linear_aligned(const float *w, int64_t in_f) {
+    return in_f % 4 == 0 && ((uintptr_t)w & 15) == 0;
+}
+
+extern "C" size_t rnn_linear_layer_workspace_size(const float *w, int64_t batch, int64_t in_f,
+                                                  int64_t out_f) {
+    return sgemm_nt_scratch(batch, out_f, in_f, linear_aligned(w, in_f));
+}
+
+extern "C" int rnn_linear_layer_ws(const float *x, int64_t batch, int64_t in_f, const float *w,
+                                   int64_t out_f, const float *bias, int relu, float *y,
+                                   void *workspace, size_t workspace_bytes, void *stream) {
     RNN_ENTRY();
     const char *name = "rnn_linear_layer";
     RNN_REQUIRE(batch >= 0 && in_f >= 0 && out_f >= 0, "%s: negative size", name);
     RNN_REQUIRE(relu == 0 || relu == 1, "%s: relu must be 0 or 1", name);
     if (batch == 0 || out_f == 0) return RNN_OK;
     RNN_REQUIRE(y != nullptr && (in_f == 0 || (x && w)), "%s: null pointer", name);
+    const size_t need = workspace ? sgemm_nt_scratch(batch, out_f, in_f, linear_aligned(w, in_f)) : 0;
+    if (need) {
+        RNN_REQUIRE(workspace_bytes >= need && ((uintptr_t)workspace & 15) == 0,
+                    "%s: workspace of %zu bytes (or misaligned), %zu needed", name, workspace_bytes,
+                    need);
+        return sgemm_nt_split(batch, out_f, in_f, x, w, bias, relu, y, workspace, as_stream(stream),
+                              name);
+    }
     // y = x . W^T with W stored [out, in] (transb = 1, ldb = in), beta = 0
     RNN_TRY(rnn_sgemm(0, 1, batch, out_f, in_f, 1.0f, x, in_f, w, in_f, 0.0f, y, out_f, stream));
     return rnn_bias_act(y, bias, batch, out_f, relu, stream);
+}
+
+extern "C" int rnn_linear_layer(const float *x, int64_t batch, int64_t in_f, const float *w,
+                                int64_t out_f, const float *bias, int relu, float *y,
+                                void *stream) {
+    return rnn_linear_layer_ws(x, batch, in_f, w, out_f, bias, relu, y, nullptr, 0, stream);
 }

@@ -19,6 +19,7 @@
 // one m and writes them as one float4.
 // Other strides / alignments take a one-thread-per-output kernel.
 #include "common.hpp"
+#include "splitgemm.hpp"
 
 namespace rnn {
 
@@ -763,6 +764,56 @@ bool aligned16f(const void *p) { return ((uintptr_t)p & 15) == 0; }
 }  // namespace rnn
 
 using namespace rnn;
+
+// ------------------------------------------------ x . W^T on split operands
+// (splitgemm.hpp). Per K step of a round of tiles: 128 x 256 2.7 us, 128 x 128
+// 1.5, 64 x 128 0.9, 64 x 64 0.52, 32 x 64 0.30, 32 x 32 0.20.
+namespace rnn {
+namespace {
+template <bool AL>
+SplitPlan nt_plan(int64_t m, int64_t n, int64_t k) {
+    using W = SplitWF32<AL>;
+    static const SplitShape shapes[] = {
+        // (the 4-byte loads' offsets leave no registers for the 128 x 256 tile)
+        split_shape<SplitCfg<W, 4, 2, AL ? 4 : 2, 4, 32>>(AL ? 2.75 : 1.6),
+        split_shape<SplitCfg<W, 4, 2, 2, 4, 32>>(1.5),
+        split_shape<SplitCfg<W, 4, 1, 2, 4, 32>>(0.87), split_shape<SplitCfg<W, 2, 1, 2, 4, 32>>(0.52),
+        split_shape<SplitCfg<W, 2, 1, 2, 2, 32>>(0.30), split_shape<SplitCfg<W, 1, 1, 2, 2, 32>>(0.20),
+    };
+    return split_plan(shapes, (int)(sizeof(shapes) / sizeof(shapes[0])), m, n, k);
+}
+bool nt_aligned(const float *w, int64_t ldw, int64_t k) {
+    return (ldw & 3) == 0 && (k & 3) == 0 && aligned16f(w);
+}
+// m <= 16 rows and 256 columns or more, aligned: the skinny kernel reads W
+// once and needs no parts. K up to 64: the f32 kernels' single launch (with
+// aligned operands; without, up to 32).
+bool nt_split_pays(int64_t m, int64_t n, int64_t k, bool aligned) {
+    if (aligned && m <= 16 && n >= 256 && k >= 32) return false;
+    return k > (aligned ? 64 : 32);
+}
+}  // namespace
+
+// Scratch bytes for x . W^T (0: the f32 kernels are used); `aligned` as the
+// operands of the call are.
+size_t sgemm_nt_scratch(int64_t m, int64_t n, int64_t k, bool aligned) {
+    if (m <= 0 || n <= 0 || !nt_split_pays(m, n, k, aligned) || !split_fits(m, k, 4 * k)) return 0;
+    return aligned ? nt_plan<true>(m, n, k).bytes : nt_plan<false>(m, n, k).bytes;
+}
+
+// y = x . W^T (+ bias, ReLU), x [m, k] and W [n, k] contiguous, in `scratch`
+// of sgemm_nt_scratch(...) bytes.
+int sgemm_nt_split(int64_t m, int64_t n, int64_t k, const float *x, const float *w, const float *bias,
+                   int relu, float *y, void *scratch, hipStream_t st, const char *name) {
+    SplitArgs a{};
+    a.x = x, a.w = w, a.c = y, a.bias = bias, a.relu = relu;
+    a.ldx = k, a.ldw = 4 * k, a.ldc = n;
+    a.M = m, a.N = n, a.K = k;
+    a.alpha = 1.0f;
+    return split_launch(nt_aligned(w, k, k) ? nt_plan<true>(m, n, k) : nt_plan<false>(m, n, k), a,
+                        scratch, st, name);
+}
+}  // namespace rnn
 
 extern "C" int rnn_sgemm(int transa, int transb, int64_t m, int64_t n, int64_t k, float alpha,
                          const float *a, int64_t lda, const float *b, int64_t ldb, float beta,

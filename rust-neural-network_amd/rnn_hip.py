@@ -95,6 +95,8 @@ SIGNATURES = {
     "rnn_w8a8_mlp": ([_P, _I64, _INT, _P, _P, _P, _P, _INT, _P, _P], _INT),
     "rnn_bias_act": ([_P, _P, _I64, _I64, _INT, _P], _INT),
     "rnn_linear_layer": ([_P, _I64, _I64, _P, _I64, _P, _INT, _P, _P], _INT),
+    "rnn_linear_layer_workspace_size": ([_P, _I64, _I64, _I64], ctypes.c_size_t),
+    "rnn_linear_layer_ws": ([_P, _I64, _I64, _P, _I64, _P, _INT, _P, _P, ctypes.c_size_t, _P], _INT),
 }
 
 _lib = None
@@ -184,6 +186,18 @@ def _dims(t, nd, name):
 def _empty(shape, dtype, like):
     import torch
     return torch.empty(shape, dtype=dtype, device=like.device)
+
+
+def _scratch(nbytes, like, stream):
+    """(device bytes for one call, or None; the call's stream), from torch's
+    allocator in the pool of that stream: freed at the end of the call, they
+    are handed out again only to work ordered behind it."""
+    import torch
+    s = _stream(stream)
+    if not nbytes:
+        return None, s
+    with torch.cuda.stream(stream):
+        return torch.empty(nbytes, dtype=torch.uint8, device=like.device), s
 
 
 # ------------------------------------------------------------------ int8
@@ -522,8 +536,10 @@ def linear_layer(x, w, bias=None, relu=False, out=None, stream=None):
     _need(bias, out_f, "bias")
     out = (_out(out, torch.float32, batch * out_f, "out") if out is not None
            else _empty((batch, out_f), torch.float32, x))
-    _check(load().rnn_linear_layer(_ptr(x), batch, in_f, _ptr(w), out_f, _ptr(bias),
-                                   int(bool(relu)), _ptr(out), _stream(stream)))
+    need = load().rnn_linear_layer_workspace_size(_ptr(w), batch, in_f, out_f)
+    ws, s = _scratch(need, x, stream)
+    _check(load().rnn_linear_layer_ws(_ptr(x), batch, in_f, _ptr(w), out_f, _ptr(bias),
+                                      int(bool(relu)), _ptr(out), _ptr(ws), need, s))
     return out
 
 
