@@ -389,6 +389,27 @@ int rnn_qt_linear_forward_ws(int format, const float *x, int64_t m, int64_t in_f
                              void *workspace, size_t workspace_bytes,
                              unsigned flags, void *stream);
 
+/* rnn_qt_linear_forward_ws with `scratch` (16-byte aligned, any contents) of
+ * at least rnn_qt_linear_scratch_size(...) bytes for calls of many rows: with
+ * it, RNN_ALGO_AUTO above 48 rows takes the cheapest of the 16-row slices, a
+ * tiled product that decodes the codes next to the bf16 MFMAs (x split exactly
+ * into three bf16 parts in the scratch; INT4, INT8, GGUF Q4_0 / Q8_0, NVFP4
+ * and BF16 weights), and dequantize + rnn_linear_layer_ws in the scratch, and
+ * allocates nothing. The size is 0 where the slices are taken (always up to
+ * 48 rows of a shape the GEMVs fit); scratch NULL: as
+ * rnn_qt_linear_forward_ws. The size depends on the alignment of data and
+ * scales. Same reference semantics (src/quantize.rs:744-754). */
+size_t rnn_qt_linear_scratch_size(int format, int64_t m, int64_t in_f,
+                                  const uint8_t *data, const float *scales,
+                                  int64_t n_scales, int64_t group, int64_t out_f);
+int rnn_qt_linear_forward_scratch(int format, const float *x, int64_t m, int64_t in_f,
+                                  const uint8_t *data, int64_t data_bytes,
+                                  const float *scales, int64_t n_scales, int64_t group,
+                                  int64_t out_f, const float *bias, float *y,
+                                  void *workspace, size_t workspace_bytes,
+                                  void *scratch, size_t scratch_bytes,
+                                  unsigned flags, void *stream);
+
 /* ------------------------------- RotorQuant KV cache + attention (next row) */
 
 /* Page sizes for `bh` sequences of `seq` positions at head dim `dim` (ng =

@@ -59,6 +59,7 @@ int device_cu_count();
 // Scratch bytes it needs, 0 where the f32 kernels are the better ones;
 // `aligned`: k % 4 == 0 and W 16-byte aligned.
 size_t sgemm_nt_scratch(int64_t m, int64_t n, int64_t k, bool aligned);
+double sgemm_nt_cost(int64_t m, int64_t n, int64_t k);  // its estimated us
 int sgemm_nt_split(int64_t m, int64_t n, int64_t k, const float *x, const float *w, const float *bias,
                    int relu, float *y, void *scratch, hipStream_t st, const char *name);
 

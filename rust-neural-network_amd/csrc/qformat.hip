@@ -8,6 +8,7 @@
 // of min(group, 32)). Codes, scales and dequantized values are bit-exact with
 // the reference; the linear forward sums in f32 in its own order.
 #include "common.hpp"
+#include "splitgemm.hpp"
 #include "numerics.hpp"
 
 namespace rnn {
@@ -1589,16 +1590,143 @@ static int gemv_kind(int format) {
     }
 }
 
+// ------------------------------------------------ more than 16 rows
+// Routes of a call that no single GEMV launch takes: 16-row slices, the tiled
+// product on split operands (splitgemm.hpp: codes decoded next to the MFMAs),
+// or dequantize + the f32 product.
+namespace rnn {
+namespace {
+
+template <int FMT>
+SplitPlan qt_tile_plan(int64_t m, int64_t n, int64_t k) {
+    using W = SplitWQ<FMT>;
+    // us per K step of a round of tiles, 4096 x 11008 and 4096 x 4096
+    static const SplitShape shapes[] = {
+        split_shape<SplitCfg<W, 4, 1, 2, 4, 32>>(0.53), split_shape<SplitCfg<W, 2, 1, 2, 2, 32>>(0.235),
+        split_shape<SplitCfg<W, 1, 1, 2, 2, 32>>(0.185),
+    };
+    return split_plan(shapes, (int)(sizeof(shapes) / sizeof(shapes[0])), m, n, k);
+}
+SplitPlan qt_tile_plan(int kind, int64_t m, int64_t n, int64_t k) {
+    switch (kind) {
+    case KIND_I4: return qt_tile_plan<SPLIT_I4>(m, n, k);
+    case KIND_I8: return qt_tile_plan<SPLIT_I8>(m, n, k);
+    case KIND_BF16: return qt_tile_plan<SPLIT_BF16>(m, n, k);
+    default: return qt_tile_plan<SPLIT_E2M1>(m, n, k);
+    }
+}
+
+// Formats whose codes bf16 holds exactly, whole 32-element steps inside a
+// group, a scale for every group, 16-byte aligned rows.
+bool qt_tile_fits(int kind, bool scaled, int64_t m, int64_t in_f, int64_t out_f, const uint8_t *data,
+                  int64_t n_scales, int64_t group) {
+    return (kind == KIND_I4 || kind == KIND_I8 || kind == KIND_BF16 || kind == KIND_E2M1) &&
+           in_f > 0 && in_f % 32 == 0 && ((uintptr_t)data & 15) == 0 &&
+           (!scaled || (group % 32 == 0 && group > 0 && (in_f % group == 0 || group % in_f == 0) &&
+                        group <= 0xffffffffLL && n_scales >= ceil_div(out_f * in_f, group))) &&
+           split_fits(m, in_f, 2 * in_f);
+}
+
+// Above this the slices are compared with the other routes (at 48 rows the
+// tiles are level with three slices of a 4096 x 4096 INT4 weight, 36 us).
+constexpr int64_t kSliceRows = 48;
+
+enum QtRoute { QT_SLICES, QT_TILES, QT_DEQUANT };
+
+// Estimated us: `per` of a 16-row slice is 4 + a time per weight of its GEMV
+// (us per 1e6 weights at 4096 x 11008: bf16 GEMV INT4 0.245, 8-bit 0.344, BF16
+// 0.37; f32 MFMA GEMV 0.49; VALU GEMV, 4 rows at a time, 1.35); dequantize 12
+// + 0.85 per 1e6 weights, the product's first reads of them included (NF4
+// 64 x 4096 x 11008: 121 us against 106 on slices). Measured at 300 x 11008 x 4096, slices or dequantize
+// against tiles: INT4 g128 280 -> 140 us, GGUF Q8_0 548 -> 143, BF16 543 -> 133.
+QtRoute qt_route(int kind, bool scaled, int64_t m, int64_t in_f, int64_t out_f, const uint8_t *data,
+                 int64_t n_scales, int64_t group, bool sliceable, double slice_rate, bool can_scratch) {
+    if (m <= kSliceRows || !can_scratch) return sliceable ? QT_SLICES : QT_DEQUANT;
+    const double mw = (double)out_f * (double)in_f * 1e-6;
+    QtRoute best = QT_DEQUANT;
+    double cost = 12.0 + 0.85 * mw;
+    const bool al = in_f % 4 == 0;
+    cost += sgemm_nt_scratch(m, out_f, in_f, al) ? sgemm_nt_cost(m, out_f, in_f)
+                                                 : 2e-9 * (double)m * (double)in_f * (double)out_f;
+    if (sliceable) {
+        const double c = (double)ceil_div(m, 16) * (4.0 + slice_rate * mw);
+        if (c < cost) best = QT_SLICES, cost = c;
+    }
+    if (qt_tile_fits(kind, scaled, m, in_f, out_f, data, n_scales, group) &&
+        qt_tile_plan(kind, m, out_f, in_f).cost < cost)
+        best = QT_TILES;
+    return best;
+}
+
+}  // namespace
+}  // namespace rnn
+
 extern "C" size_t rnn_qt_linear_workspace_size(int64_t in_f, int64_t out_f) {
     return in_f > 0 && out_f > 0 ? bf16_workspace(out_f) : 0;
 }
 
-extern "C" int rnn_qt_linear_forward_ws(int format, const float *x, int64_t m, int64_t in_f,
-                                        const uint8_t *data, int64_t data_bytes,
-                                        const float *scales, int64_t n_scales, int64_t group,
-                                        int64_t out_f, const float *bias, float *y,
-                                        void *workspace, size_t workspace_bytes, unsigned flags,
-                                        void *stream) {
+// What of a format's GEMVs a shape admits (the conditions of the forward).
+struct QtGemvs {
+    int kind, ep;
+    bool scaled, fits, mfma, bf16;  // VALU; f32 MFMA; bf16 MFMA (<= 16 rows)
+    int64_t slice_limit;            // rows that AUTO slices without scratch
+    double slice_rate;              // us per 1e6 weights of a 16-row slice
+};
+static QtGemvs qt_gemvs(int format, int64_t rows, int64_t in_f, const uint8_t *data,
+                        const float *scales, int64_t n_scales, int64_t group, int64_t out_f,
+                        bool x_aligned) {
+    QtGemvs g;
+    g.kind = gemv_kind(format);
+    g.scaled = format != RNN_QF_FP16 && format != RNN_QF_BF16;
+    g.ep = g.kind >= 0 ? piece_elems(g.kind) : 32;
+    g.fits = g.kind >= 0 && in_f % 32 == 0 &&
+             (!g.scaled || (group % (kind4(g.kind) ? 32 : 16) == 0 && group <= 0xffffffffLL &&
+                            (in_f % group == 0 || group % in_f == 0))) &&
+             x_aligned && ((uintptr_t)data % 16) == 0 && out_f <= 0x7fffffffLL;
+    // the f32 MFMA GEMV takes all rows at once; its 4 waves split K in whole
+    // chunks of 4 pieces
+    g.mfma = g.fits && rows <= 16 && in_f % (kMfmaWaves * 4 * g.ep) == 0;
+    // the bf16 MFMA GEMV: integer codes and bf16 weights, whole chunks of
+    // 4 pieces per group
+    g.bf16 = g.fits && rows <= 16 && (g.kind == KIND_I4 || g.kind == KIND_I8 || g.kind == KIND_BF16) &&
+             in_f % (kBf16Waves * 4 * g.ep) == 0 &&
+             (!g.scaled || (group % (4 * g.ep) == 0 && in_f % group == 0) || group % in_f == 0 ||
+              // (groups of 32: a chunk's scales come in one vector load)
+              (group == 32 && g.kind != KIND_BF16 && ((uintptr_t)scales % 16) == 0)) &&
+             // (a scale for every group: the kernel reads a row's scales from the
+             // row's first without the per-index clamp of a shortened array)
+             (!g.scaled || n_scales >= ceil_div(out_f * in_f, group)) &&
+             bf16_plan(rows, in_f, out_f, g.ep).S > 0 && 64 * in_f * 16 / g.ep < (int64_t(1) << 31) &&
+             16 * in_f * 4 < (int64_t(1) << 31);
+    g.slice_limit = g.bf16 ? (g.kind == KIND_I4 ? 512 : 192) : g.mfma ? 96 : 32;
+    g.slice_rate = g.bf16 ? (g.kind == KIND_I4 ? 0.245 : g.kind == KIND_I8 ? 0.344 : 0.37)
+                   : g.mfma ? 0.49
+                            : 1.35;
+    return g;
+}
+
+extern "C" size_t rnn_qt_linear_scratch_size(int format, int64_t m, int64_t in_f, const uint8_t *data,
+                                             const float *scales, int64_t n_scales, int64_t group,
+                                             int64_t out_f) {
+    if (m <= 16 || in_f <= 0 || out_f <= 0 || (format != RNN_QF_FP16 && format != RNN_QF_BF16 && group <= 0))
+        return 0;
+    const QtGemvs g = qt_gemvs(format, 16, in_f, data, scales, n_scales, group, out_f, true);
+    switch (qt_route(g.kind, g.scaled, m, in_f, out_f, data, n_scales, group, g.fits, g.slice_rate, true)) {
+    case QT_SLICES: return 0;
+    case QT_TILES: return qt_tile_plan(g.kind, m, out_f, in_f).bytes;
+    default: {
+        const size_t w = ((size_t)out_f * (size_t)in_f * 4 + 255) / 256 * 256;
+        return w + sgemm_nt_scratch(m, out_f, in_f, in_f % 4 == 0);
+    }
+    }
+}
+
+extern "C" int rnn_qt_linear_forward_scratch(int format, const float *x, int64_t m, int64_t in_f,
+                                             const uint8_t *data, int64_t data_bytes,
+                                             const float *scales, int64_t n_scales, int64_t group,
+                                             int64_t out_f, const float *bias, float *y,
+                                             void *workspace, size_t workspace_bytes, void *scratch,
+                                             size_t scratch_bytes, unsigned flags, void *stream) {
     RNN_ENTRY();
     const char *name = "rnn_qt_linear_forward";
     RNN_REQUIRE(!workspace || (workspace_bytes >= rnn_qt_linear_workspace_size(in_f, out_f) &&
@@ -1620,50 +1748,61 @@ extern "C" int rnn_qt_linear_forward_ws(int format, const float *x, int64_t m, i
         if (bias) qt_bias_kernel<<<grid_for(m * out_f, 256), 256, 0, st>>>(y, m, out_f, bias);
         return check_launch(name);
     }
-    const int kind = gemv_kind(format);
-    const bool scaled = format != RNN_QF_FP16 && format != RNN_QF_BF16;
-    const bool fits = kind >= 0 && in_f % 32 == 0 &&
-                      (!scaled || (group % (kind4(kind) ? 32 : 16) == 0 && group <= 0xffffffffLL &&
-                                   (in_f % group == 0 || group % in_f == 0))) &&
-                      ((uintptr_t)x % 16) == 0 && ((uintptr_t)data % 16) == 0 &&
-                      out_f <= 0x7fffffffLL;
-    // the MFMA GEMV takes all m <= 16 rows at once; its 4 waves split K in
-    // whole chunks of 4 pieces
-    const bool fits_mfma = fits && m <= 16 && in_f % (kMfmaWaves * 4 * piece_elems(kind)) == 0;
-    // the bf16 MFMA GEMV: integer codes and bf16 weights, whole chunks of
-    // 4 pieces per group
-    const int ep = kind >= 0 ? piece_elems(kind) : 32;
-    auto bf16_fits = [&](int64_t rows) {
-        return fits && rows <= 16 && (kind == KIND_I4 || kind == KIND_I8 || kind == KIND_BF16) &&
-        in_f % (kBf16Waves * 4 * ep) == 0 &&
-        (!scaled || (group % (4 * ep) == 0 && in_f % group == 0) || group % in_f == 0 ||
-         // (groups of 32: a chunk's scales come in one vector load)
-         (group == 32 && kind != KIND_BF16 && ((uintptr_t)scales % 16) == 0)) &&
-        // (a scale for every group: the kernel reads a row's scales from the
-        // row's first without the per-index clamp of a shortened array)
-        (!scaled || n_scales >= ceil_div(out_f * in_f, group)) &&
-        bf16_plan(rows, in_f, out_f, ep).S > 0 && 64 * in_f * 16 / ep < (int64_t(1) << 31) &&
-        16 * in_f * 4 < (int64_t(1) << 31);
-    };
-    const bool fits_bf16 = bf16_fits(m);
-    // m > 16: the GEMVs run on 16-row slices of x and y, one after the other,
-    // each slice reading the weights again. A forced GEMV does so for every
-    // m; AUTO does so while the slices beat dequantize + f32 GEMM (measured,
+    const QtGemvs gv = qt_gemvs(format, m, in_f, data, scales, n_scales, group, out_f,
+                                ((uintptr_t)x % 16) == 0);
+    const int kind = gv.kind, ep = gv.ep;
+    const bool fits = gv.fits, fits_mfma = gv.mfma, fits_bf16 = gv.bf16;
+    // m > 16 with scratch: the cheapest route; the sizes behind the scratch
+    // are recomputed here, so a scratch of another shape is refused
+    const size_t need = scratch && algo == RNN_ALGO_AUTO
+                            ? rnn_qt_linear_scratch_size(format, m, in_f, data, scales, n_scales, group, out_f)
+                            : 0;
+    bool slice = m > 16 && algo != RNN_ALGO_TILED;
+    if (need) {
+        RNN_REQUIRE(scratch_bytes >= need && ((uintptr_t)scratch % 16) == 0,
+                    "%s: scratch of %zu bytes (or misaligned), %zu needed", name, scratch_bytes, need);
+        const QtGemvs g16 = qt_gemvs(format, 16, in_f, data, scales, n_scales, group, out_f, true);
+        const QtRoute r = qt_route(kind, gv.scaled, m, in_f, out_f, data, n_scales, group, g16.fits,
+                                   g16.slice_rate, true);
+        SplitArgs a{};
+        if (r == QT_TILES) {
+            a.x = x, a.w = data, a.scales = scales, a.bias = bias, a.c = y;
+            a.ldx = in_f, a.ldw = kind4(kind) ? in_f / 2 : kind == KIND_I8 ? in_f : 2 * in_f;
+            a.ldc = out_f, a.M = m, a.N = out_f, a.K = in_f, a.alpha = 1.0f;
+            a.sc_n = 1, a.sc_d = 1;
+            if (gv.scaled && in_f % group == 0)
+                a.sc_n = in_f / group, a.sc_k = (uint32_t)(group / 32);
+            else if (gv.scaled)
+                a.sc_d = group / in_f;
+            return split_launch(qt_tile_plan(kind, m, out_f, in_f), a, scratch, st, name);
+        }
+        // dequantize() into the scratch, then x . W^T + bias
+        const size_t wb = ((size_t)out_f * (size_t)in_f * 4 + 255) / 256 * 256;
+        float *w = static_cast<float *>(scratch);
+        RNN_TRY(rnn_qt_dequantize(format, data, data_bytes, scales, n_scales, group, out_f * in_f, w,
+                                  stream));
+        return rnn_linear_layer_ws(x, m, in_f, w, out_f, bias, 0, y,
+                                   need > wb ? static_cast<uint8_t *>(scratch) + wb : nullptr, need - wb,
+                                   stream);
+    }
+    // Without scratch, or where the slices are the cheapest: the GEMVs run on
+    // 16-row slices of x and y, one after the other, each slice reading the
+    // weights again. A forced GEMV does so for every m; AUTO does so while the
+    // slices beat dequantize + f32 GEMM (measured,
     // 4096 x 11008, slices against the latter: bf16 GEMV INT4 g128 m = 32
     // 29.9 us against 182, m = 512 467 against 554; GGUF Q8_0 m = 192 232
     // against 327, m = 256 316 against 306; BF16 m = 192 249 against 341,
     // m = 256 305 against 291; f32 MFMA GEMV NF4 g64 m = 96 157 against 178,
     // m = 128 208 against 194)
-    if (m > 16 && algo != RNN_ALGO_TILED) {
-        const int64_t lim = bf16_fits(16) ? (kind == KIND_I4 ? 512 : 192)
-                            : fits && in_f % (kMfmaWaves * 4 * ep) == 0 ? 96
-                                                                        : 32;
-        if (algo != RNN_ALGO_AUTO || (fits && m <= lim)) {
+    if (slice) {
+        const QtGemvs g16 = qt_gemvs(format, 16, in_f, data, scales, n_scales, group, out_f,
+                                     ((uintptr_t)x % 16) == 0);
+        if (algo != RNN_ALGO_AUTO || (fits && (m <= g16.slice_limit || scratch))) {
             for (int64_t m0 = 0; m0 < m; m0 += 16)
-                RNN_TRY(rnn_qt_linear_forward_ws(format, x + m0 * in_f, std::min<int64_t>(16, m - m0), in_f,
-                                                 data, data_bytes, scales, n_scales, group, out_f,
-                                                 bias, y + m0 * out_f, workspace, workspace_bytes,
-                                                 flags, stream));
+                RNN_TRY(rnn_qt_linear_forward_scratch(
+                    format, x + m0 * in_f, std::min<int64_t>(16, m - m0), in_f, data, data_bytes, scales,
+                    n_scales, group, out_f, bias, y + m0 * out_f, workspace, workspace_bytes, nullptr, 0,
+                    flags, stream));
             return RNN_OK;
         }
     }
@@ -1753,6 +1892,17 @@ extern "C" int rnn_qt_linear_forward_ws(int format, const float *x, int64_t m, i
     }
     const int rf = check_hip(hipFreeAsync(w, st), name);
     return rc != RNN_OK ? rc : rf;
+}
+
+extern "C" int rnn_qt_linear_forward_ws(int format, const float *x, int64_t m, int64_t in_f,
+                                        const uint8_t *data, int64_t data_bytes,
+                                        const float *scales, int64_t n_scales, int64_t group,
+                                        int64_t out_f, const float *bias, float *y,
+                                        void *workspace, size_t workspace_bytes, unsigned flags,
+                                        void *stream) {
+    return rnn_qt_linear_forward_scratch(format, x, m, in_f, data, data_bytes, scales, n_scales, group,
+                                         out_f, bias, y, workspace, workspace_bytes, nullptr, 0, flags,
+                                         stream);
 }
 
 extern "C" int rnn_qt_linear_forward(int format, const float *x, int64_t m, int64_t in_f,

@@ -801,6 +801,9 @@ size_t sgemm_nt_scratch(int64_t m, int64_t n, int64_t k, bool aligned) {
     return aligned ? nt_plan<true>(m, n, k).bytes : nt_plan<false>(m, n, k).bytes;
 }
 
+// The estimate behind the choice of its tiles (us).
+double sgemm_nt_cost(int64_t m, int64_t n, int64_t k) { return nt_plan<true>(m, n, k).cost; }
+
 // y = x . W^T (+ bias, ReLU), x [m, k] and W [n, k] contiguous, in `scratch`
 // of sgemm_nt_scratch(...) bytes.
 int sgemm_nt_split(int64_t m, int64_t n, int64_t k, const float *x, const float *w, const float *bias,

@@ -540,7 +540,7 @@ void split_gemm_kernel(SplitArgs a) {
 
 // C = alpha * (P_0 + ... + P_{S-1}) + beta * C (+ bias, ReLU): the ranges'
 // partial products (M x N each, cstride apart) added in order.
-__global__ __launch_bounds__(256) void split_sum_kernel(const float *__restrict__ P, int S,
+static __global__ __launch_bounds__(256) void split_sum_kernel(const float *__restrict__ P, int S,
                                                         SplitArgs a) {
     for (int64_t m = blockIdx.y; m < a.M; m += gridDim.y)
         for (int64_t n = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; n < a.N;

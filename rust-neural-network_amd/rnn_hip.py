@@ -85,6 +85,9 @@ SIGNATURES = {
                                         ctypes.c_float, _P, _P, ctypes.c_size_t, _P], _INT),
     "rnn_qt_linear_forward_ws": ([_INT, _P, _I64, _I64, _P, _I64, _P, _I64, _I64, _I64, _P, _P,
                                   _P, ctypes.c_size_t, _UINT, _P], _INT),
+    "rnn_qt_linear_scratch_size": ([_INT, _I64, _I64, _P, _P, _I64, _I64, _I64], ctypes.c_size_t),
+    "rnn_qt_linear_forward_scratch": ([_INT, _P, _I64, _I64, _P, _I64, _P, _I64, _I64, _I64, _P, _P,
+                                       _P, ctypes.c_size_t, _P, ctypes.c_size_t, _UINT, _P], _INT),
     "rnn_rotorquant_kv_page_elems": ([_I64, _I64, _I64, _P, _P], _INT),
     "rnn_rotorquant_kv_pack": ([_P, _P, _I64, _I64, _I64, _INT, _INT, _P, _P, _P], _INT),
     "rnn_rotorquant_kv_attention": ([_P, _I64, _I64, _P, _P, _P, _P, _P, _P, _I64, _I64,
@@ -607,10 +610,13 @@ def qt_linear_forward(fmt, x, data, scales, group, out_f, bias=None, algo=ALGO_A
     _need(bias, out_f, "bias")
     y = _out(y, torch.float32, m * out_f, "y") if y is not None else _empty((m, out_f), torch.float32, x)
     ws_bytes = 0 if workspace is None else workspace.numel()
-    _check(load().rnn_qt_linear_forward_ws(fmt, _ptr(x), m, in_f, _ptr(data), data.numel(),
-                                           _ptr(scales), scales.numel(), group, out_f, _ptr(bias),
-                                           _ptr(y), _ptr(workspace), ws_bytes, algo,
-                                           _stream(stream)))
+    need = (load().rnn_qt_linear_scratch_size(fmt, m, in_f, _ptr(data), _ptr(scales), scales.numel(),
+                                              group, out_f) if m > 16 and algo == ALGO_AUTO else 0)
+    scratch, s = _scratch(need, x, stream)
+    _check(load().rnn_qt_linear_forward_scratch(fmt, _ptr(x), m, in_f, _ptr(data), data.numel(),
+                                                _ptr(scales), scales.numel(), group, out_f,
+                                                _ptr(bias), _ptr(y), _ptr(workspace), ws_bytes,
+                                                _ptr(scratch), need, algo, s))
     return y
 
 

@@ -121,3 +121,77 @@ def test_linear_layer_split_capture_and_streams(dev, hip):
         x.mul_(1.5)
         g.replay()
         assert torch.equal(out, hip.linear_layer(x, w, b)), i
+
+
+FORMATS = {"INT4-g128": (H.QF_INT4, 128), "Q4_0": (H.QF_GGUF_Q4, 32), "INT8-g64": (H.QF_INT8, 64),
+           "Q8_0": (H.QF_GGUF_Q8, 32), "BF16": (H.QF_BF16, 0), "NVFP4-g32": (H.QF_NVFP4, 32),
+           "INT8-rows": (H.QF_INT8, 1024), "INT4-tensor": (H.QF_INT4, 0), "INT8-2rows": (H.QF_INT8, 2048)}
+
+
+def quantized(fmt, gs, n, k, seed):
+    import torch
+    g = torch.Generator(device="cuda").manual_seed(seed)
+    w = torch.randn((n, k), generator=g, device="cuda") * 0.02
+    d, s, gg = H.qt_quantize(fmt, w, gs if gs else n * k)
+    return d, s, gg, H.qt_dequantize(fmt, d, s, gg, n * k).view(n, k)
+
+
+# tiles of 32x32, 32x64 and 64x128, one and several ranges of K, ragged m and n
+@pytest.mark.parametrize("m,k,n", [(49, 1024, 33), (300, 1024, 2049), (130, 4096, 1000),
+                                   (1000, 1024, 4096), (65, 11264, 64)])
+@pytest.mark.parametrize("name", FORMATS)
+def test_quantized_linear_tiles(dev, hip, name, m, k, n):
+    import torch
+    fmt, gs = FORMATS[name]
+    if gs > 32 and (k % gs and gs % k):
+        pytest.skip("a group that neither divides nor is divided by a row")
+    if gs == 2048 and n % 2:
+        n += 1
+    d, s, g, w = quantized(fmt, gs, n, k, m + n)
+    x, _, b = data(m, k, n, m)
+    size = hip.load().rnn_qt_linear_scratch_size(fmt, m, k, d.data_ptr(), s.data_ptr(), s.numel(), g, n)
+    parts = -(-m // 128) * 128 * -(-k // 32) * 192 + 8 * 4 * m * n
+    assert 0 <= size <= parts                           # the tiles' scratch (or the slices': none)
+    y = torch.full((m * n + 16,), -5.0, device="cuda")
+    out = y[:m * n].view(m, n)
+    hip.qt_linear_forward(fmt, x, d, s, g, n, b, y=out)
+    check(out, x, w, b)
+    assert bool((y[m * n:] == -5).all())
+    assert torch.equal(out, hip.qt_linear_forward(fmt, x, d, s, g, n, b))
+
+
+@pytest.mark.parametrize("name", ["INT4-g128", "Q8_0", "BF16", "NVFP4-g32"])
+def test_quantized_linear_tiles_nonfinite(dev, hip, name):
+    """Non-finite x, scales and BF16 weights, and x below bf16's range, on the
+    tiles: the pattern of the f32 product of the dequantized weight."""
+    import torch
+    fmt, gs = FORMATS[name]
+    m, k, n = 200, 1024, 700
+    d, s, g, _ = quantized(fmt, gs, n, k, 3)
+    x, _, _ = data(m, k, n, 4)
+    x[1, 5], x[3, 6], x[70, 9] = float("inf"), float("nan"), 2.0 ** -130
+    x[90] *= 2.0 ** -115
+    if name == "BF16":
+        d.view(torch.int16)[11 * k + 7] = 0x7F80        # +inf
+        d.view(torch.int16)[12 * k + 7] = 0x7FC0        # NaN
+    else:
+        s[11 * k // g] = float("inf")
+    w = hip.qt_dequantize(fmt, d, s, g, n * k).view(n, k)
+    assert hip.load().rnn_qt_linear_scratch_size(fmt, m, k, d.data_ptr(), s.data_ptr(), s.numel(), g, n) > 0
+    y = hip.qt_linear_forward(fmt, x, d, s, g, n)
+    ref = x.double() @ w.double().t()
+    assert torch.equal(torch.isnan(y), torch.isnan(ref)) and torch.equal(torch.isinf(y), torch.isinf(ref))
+    fine = torch.isfinite(ref)
+    lim = (k + 4) * U * (x.nan_to_num(0, 0, 0).double().abs() @ w.nan_to_num(0, 0, 0).double().abs().t())
+    assert bool(((y.double() - ref).abs() <= lim + k * 2.0 ** -149)[fine].all())
+
+
+def test_quantized_linear_dequantize_in_scratch(dev, hip):
+    """Formats and groups the tiles do not take, m above the slices: the weight
+    is dequantized into the call's scratch."""
+    import torch
+    for fmt, gs, m, k, n in ((H.QF_NF4, 64, 700, 512, 300), (H.QF_FP16, 0, 700, 512, 300),
+                             (H.QF_INT4, 33, 100, 201, 70), (H.QF_NF4, 64, 20, 200, 70)):
+        d, s, g, w = quantized(fmt, gs, n, k, m)
+        x, _, b = data(m, k, n, m)
+        check(hip.qt_linear_forward(fmt, x, d, s, g, n, b), x, w, b)
