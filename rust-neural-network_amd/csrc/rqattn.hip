@@ -95,6 +95,15 @@ __device__ __forceinline__ float rq_code(uint32_t w, int c) {
     return (float)(((int32_t)(w << (28 - 4 * c))) >> 28);
 }
 
+// The three codes of group `odd` (0 or 1) of a pair of group words, each as
+// c / 16: v_cvt_off_f32_i4 reads the low 4 bits of a selected byte as a signed
+// value, so a pair takes one shift and six conversions. h = w >> 4.
+__device__ __forceinline__ void rq_codes16(uint32_t w, uint32_t h, int odd, float (&c)[3]) {
+    c[0] = __builtin_amdgcn_cvt_off_f32_i4((int)((odd ? w >> 16 : w) & 0xFFu));
+    c[1] = __builtin_amdgcn_cvt_off_f32_i4((int)((odd ? h >> 16 : h) & 0xFFu));
+    c[2] = __builtin_amdgcn_cvt_off_f32_i4((int)((odd ? w >> 24 : w >> 8) & 0xFFu));
+}
+
 __device__ __forceinline__ float wave_max_f(float v) {
 #pragma unroll
     for (int off = 32; off > 0; off >>= 1) v = fmaxf(v, __shfl_xor(v, off, 64));
@@ -157,8 +166,10 @@ __device__ __forceinline__ void rq_load_k(RqTileK<NG4, NG8> &t, const uint16_t *
 }
 
 
-// grid: (BH * nq, splits) workgroups of kAttnWaves waves; ng <= 4 * NG4 <= 8
-// * NG8 <= 64. Split y takes tiles [y * tps, min(T, (y + 1) * tps)). With
+// grid: (BH * ceil(nq / NQ), splits) workgroups of kAttnWaves waves; ng <= 4 *
+// NG4 <= 8 * NG8 <= 64. A workgroup takes up to NQ queries of one sequence
+// (rows past nq repeat the last query and are not stored): each page tile is
+// read and its codes converted once for all of them. Split y takes tiles [y * tps, min(T, (y + 1) * tps)). With
 // several splits (part != null) each writes its unnormalised state (max,
 // sum, rotated accumulators) to part and counts itself in at cnt[query];
 // the last of a query's splits merges the states in split order (M = max
@@ -168,18 +179,21 @@ __device__ __forceinline__ void rq_load_k(RqTileK<NG4, NG8> &t, const uint16_t *
 // to the device's coherence point and complete (vmcnt 0) before the count;
 // the last split reads them with device-scope atomic loads. No workgroup
 // waits for another.
-template <int NG4, int NG8>
-__global__ __launch_bounds__(kAttnWaves * 64) void rq_kv_attn_kernel(
+template <int NG4, int NG8, int NQ>
+__global__ __launch_bounds__(kAttnWaves * 64)
+__attribute__((amdgpu_waves_per_eu(NQ == 1 && NG4 <= 11 ? 2 : 1)))
+void rq_kv_attn_kernel(
     const float *__restrict__ q, const uint16_t *__restrict__ kc, const float *__restrict__ ks,
     const uint16_t *__restrict__ vc, const float *__restrict__ vs, const float *__restrict__ krot,
     const float *__restrict__ vrot, int64_t nq, int64_t S, int64_t dim, int64_t ng, int64_t T,
     int64_t tps, float scale, float *__restrict__ out, float *__restrict__ part,
     uint32_t *__restrict__ cnt) {
-    __shared__ __attribute__((aligned(16))) float qs[4 * 64];  // rotated query, 4 floats per group
-    __shared__ __attribute__((aligned(16))) float pb[kAttnWaves][64];
-    __shared__ float mrg[kAttnWaves][2 + 3 * 64];
+    __shared__ __attribute__((aligned(16))) float qs[NQ][4 * 64];  // rotated queries, 4 floats per group
+    __shared__ __attribute__((aligned(16))) float pb[kAttnWaves][NQ][64];
+    __shared__ float mrg[NQ][kAttnWaves][2 + 3 * 64];
     const int wid = threadIdx.x / 64, lane = threadIdx.x % 64;
-    const int64_t bh = blockIdx.x / nq, qi = blockIdx.x % nq;
+    const int64_t nqb = (nq + NQ - 1) / NQ;
+    const int64_t bh = blockIdx.x / nqb, q0 = blockIdx.x % nqb * NQ;
     const int g = lane < ng ? lane : (int)ng - 1;  // group lanes past ng mirror the last one
     const bool gact = lane < ng;
 
@@ -197,10 +211,10 @@ __global__ __launch_bounds__(kAttnWaves * 64) void rq_kv_attn_kernel(
     }
 
     // rotated query q'_g = R_g q_g (zero past dim), published in LDS
-    if (wid == 0) {
+    for (int qq = wid; qq < NQ; qq += kAttnWaves) {
         float R[9];
         rotation_matrix(krot + 4 * g, R);
-        const float *qrow = q + (bh * nq + qi) * dim;
+        const float *qrow = q + (bh * nq + (q0 + qq < nq ? q0 + qq : nq - 1)) * dim;
         float x[3];
 #pragma unroll
         for (int c = 0; c < 3; ++c) {  // unconditional load (index clamped), zero past dim
@@ -213,83 +227,113 @@ __global__ __launch_bounds__(kAttnWaves * 64) void rq_kv_attn_kernel(
         for (int i = 0; i < 3; ++i)
             qv[i] = gact ? R[3 * i] * x[0] + R[3 * i + 1] * x[1] + R[3 * i + 2] * x[2] : 0.0f;
         qv[3] = 0.0f;
-        *reinterpret_cast<f4v *>(&qs[4 * lane]) = qv;
+        *reinterpret_cast<f4v *>(&qs[qq][4 * lane]) = qv;
     }
     // a barrier over LDS only: the tile loads stay in flight
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
-    float m = -INFINITY, l = 0.0f, a0 = 0.0f, a1 = 0.0f, a2 = 0.0f;
+    const float scale16 = 16.0f * scale;  // (the sums are of c / 16: the same rounding)
+    float m[NQ], l[NQ], acc[NQ][3];
+#pragma unroll
+    for (int qq = 0; qq < NQ; ++qq)
+        m[qq] = -INFINITY, l[qq] = acc[qq][0] = acc[qq][1] = acc[qq][2] = 0.0f;
     for (int64_t i = 0; i < nt; ++i) {
         const int64_t t = tb + wid + i * kAttnWaves;
         // the next tile, or this one again at the end (an L2 hit): the loads
         // stay unconditional so that the compiler's waits stay exact
         const int64_t tn = t + kAttnWaves <= last ? t + kAttnWaves : t;
         // lane = position: score = scale * sum_g s_g (q'_g . c_g)
-        float sc = 0.0f;
+        float sc[NQ];
+#pragma unroll
+        for (int qq = 0; qq < NQ; ++qq) sc[qq] = 0.0f;
 #pragma unroll
         for (int gg = 0; gg < 4 * NG4; ++gg) {
-            const f4v qv = *reinterpret_cast<const f4v *>(&qs[4 * (gg < ng ? gg : 0)]);
             const uint32_t word = (uint32_t)K.c[gg / 8][(gg % 8) / 2];
-            const uint32_t w = (gg & 1) ? (word >> 16) : word;
-            float d = qv[0] * rq_code(w, 0);
-            d = __builtin_fmaf(qv[1], rq_code(w, 1), d);
-            d = __builtin_fmaf(qv[2], rq_code(w, 2), d);
+            uint32_t h = word >> 4;
+            if (NQ > 1) asm("" : "+v"(h));  // a register of its own, whose bytes the conversions select
+            float c[3];
+            rq_codes16(word, h, gg & 1, c);
             const float sg = gg < ng ? K.s[gg / 4][gg % 4] : 0.0f;
-            sc = __builtin_fmaf(sg, d, sc);
+#pragma unroll
+            for (int qq = 0; qq < NQ; ++qq) {
+                const f4v qv = *reinterpret_cast<const f4v *>(&qs[qq][4 * (gg < ng ? gg : 0)]);
+                float d = qv[0] * c[0];
+                d = __builtin_fmaf(qv[1], c[1], d);
+                d = __builtin_fmaf(qv[2], c[2], d);
+                sc[qq] = __builtin_fmaf(sg, d, sc[qq]);
+            }
         }
         rq_load_k<NG4, NG8>(K, kc, ks, seq + tn, ng, lane);
-        sc *= scale;
-        if (t * kTile + lane >= S) sc = -INFINITY;
-        const float mt = wave_max_f(sc);
-        const float mn = fmaxf(m, mt);
-        const float corr = expf(m - mn);  // 0 on the first tile (m = -inf)
-        const float p = expf(sc - mn);    // 0 for masked positions
-        l = l * corr + p;
-        m = mn;
-        pb[wid][lane] = p;
+#pragma unroll
+        for (int qq = 0; qq < NQ; ++qq) {
+            float s = sc[qq] * scale16;
+            if (t * kTile + lane >= S) s = -INFINITY;
+            const float mt = wave_max_f(s);
+            const float mn = fmaxf(m[qq], mt);
+            const float corr = expf(m[qq] - mn);  // 0 on the first tile (m = -inf)
+            const float p = expf(s - mn);         // 0 for masked positions
+            l[qq] = l[qq] * corr + p;
+            m[qq] = mn;
+            pb[wid][qq][lane] = p;
+#pragma unroll
+            for (int c = 0; c < 3; ++c) acc[qq][c] *= corr;
+        }
         __builtin_amdgcn_wave_barrier();  // one wave's LDS operations complete in order
         // lane = group: acc_g = acc_g * corr + sum_j p_j s_jg c_jg (rotated domain)
-        a0 *= corr, a1 *= corr, a2 *= corr;
 #pragma unroll
         for (int q4 = 0; q4 < 16; ++q4) {
-            const f4v p4 = *reinterpret_cast<const f4v *>(&pb[wid][4 * q4]);
+            f4v p4[NQ];
+#pragma unroll
+            for (int qq = 0; qq < NQ; ++qq) p4[qq] = *reinterpret_cast<const f4v *>(&pb[wid][qq][4 * q4]);
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
                 const uint32_t word = (uint32_t)V.c[q4 / 2][2 * (q4 & 1) + r / 2];
-                const uint32_t w = (r & 1) ? (word >> 16) : (word & 0xFFFFu);
-                const float ws = p4[r] * V.s[q4][r];
-                a0 = __builtin_fmaf(ws, rq_code(w, 0), a0);
-                a1 = __builtin_fmaf(ws, rq_code(w, 1), a1);
-                a2 = __builtin_fmaf(ws, rq_code(w, 2), a2);
+                uint32_t h = word >> 4;
+                if (NQ > 1) asm("" : "+v"(h));
+                float c[3];
+                rq_codes16(word, h, r & 1, c);
+#pragma unroll
+                for (int qq = 0; qq < NQ; ++qq) {
+                    const float ws = p4[qq][r] * V.s[q4][r];
+#pragma unroll
+                    for (int i = 0; i < 3; ++i) acc[qq][i] = __builtin_fmaf(ws, c[i], acc[qq][i]);
+                }
             }
         }
         rq_load_v(V, vc, vs, seq + tn, ng, g);
         __builtin_amdgcn_wave_barrier();
     }
-    // merge the waves: M = max m_w, L = sum l_w e^(m_w - M), A = sum a_w e^(m_w - M)
-    l = wave_sum_f(l);
-    if (lane == 0) mrg[wid][0] = m, mrg[wid][1] = l;
-    mrg[wid][2 + 3 * lane] = a0, mrg[wid][3 + 3 * lane] = a1, mrg[wid][4 + 3 * lane] = a2;
+    // merge the waves, a wave per query: M = max m_w, L = sum l_w e^(m_w - M),
+    // A = sum a_w e^(m_w - M)
+#pragma unroll
+    for (int qq = 0; qq < NQ; ++qq) {
+        const float lw = wave_sum_f(l[qq]);
+        if (lane == 0) mrg[qq][wid][0] = m[qq], mrg[qq][wid][1] = lw;
+#pragma unroll
+        for (int c = 0; c < 3; ++c) mrg[qq][wid][2 + 3 * lane + c] = 16.0f * acc[qq][c];
+    }
     __syncthreads();
-    if (wid != 0) return;
+    if (wid >= NQ || q0 + wid >= nq) return;
+    const float (*const mw_)[2 + 3 * 64] = mrg[wid];
+    const int64_t qrow = bh * nq + q0 + wid;
     float M = -INFINITY;
 #pragma unroll
-    for (int w = 0; w < kAttnWaves; ++w) M = fmaxf(M, mrg[w][0]);
+    for (int w = 0; w < kAttnWaves; ++w) M = fmaxf(M, mw_[w][0]);
     float L = 0.0f, A0 = 0.0f, A1 = 0.0f, A2 = 0.0f;
     if (M != -INFINITY) {
 #pragma unroll
         for (int w = 0; w < kAttnWaves; ++w) {
-            const float mw = mrg[w][0];
+            const float mw = mw_[w][0];
             const float f = mw == -INFINITY ? 0.0f : expf(mw - M);
-            L = L + f * mrg[w][1];
-            A0 = A0 + f * mrg[w][2 + 3 * lane];
-            A1 = A1 + f * mrg[w][3 + 3 * lane];
-            A2 = A2 + f * mrg[w][4 + 3 * lane];
+            L = L + f * mw_[w][1];
+            A0 = A0 + f * mw_[w][2 + 3 * lane];
+            A1 = A1 + f * mw_[w][3 + 3 * lane];
+            A2 = A2 + f * mw_[w][4 + 3 * lane];
         }
     }
     if (part) {
-        const int64_t qrow = bh * nq + qi, stride = 2 + 3 * ng;
+        const int64_t stride = 2 + 3 * ng;
         const int ns = (int)gridDim.y;
         float *pp = part + (qrow * ns + blockIdx.y) * stride;
         if (lane == 0) {
@@ -339,7 +383,7 @@ __global__ __launch_bounds__(kAttnWaves * 64) void rq_kv_attn_kernel(
     if (!gact) return;
     float R[9];
     rotation_matrix(vrot + 4 * g, R);
-    float *orow = out + (bh * nq + qi) * dim;
+    float *orow = out + qrow * dim;
 #pragma unroll
     for (int c = 0; c < 3; ++c) {
         const float o = (R[c] * A0 + R[3 + c] * A1 + R[6 + c] * A2) * inv;  // R^T A, then * inv
@@ -585,18 +629,37 @@ static void attn_splits(int64_t wgs, int64_t T, bool wide, int64_t &ns, int64_t 
 // Split workspace: the counts (one per query and range), then the splits'
 // states [query][split][2 + 3 ng]. The counts' area is the same for every
 // shape -- a call splits only while its workgroups number fewer than
-// kWideWgsPerCu per CU (attn_splits) -- so a workspace left by one shape holds
-// zeros where another shape's counts are.
+// kNarrowWgsPerCu (of up to kMaxGroup queries) or kWideWgsPerCu per CU
+// (attn_splits) -- so a workspace left by one shape holds zeros where another
+// shape's counts are.
+constexpr int kMaxGroup = 4;
+static_assert(kMaxGroup <= kAttnWaves, "a wave per query merges the states");
 static size_t attn_count_bytes() {
-    return (size_t)ceil_div(4 * (int64_t)kWideWgsPerCu * device_cu_count(), 256) * 256;
+    const int64_t per_cu = std::max(kNarrowWgsPerCu * kMaxGroup, kWideWgsPerCu);
+    return (size_t)ceil_div(4 * per_cu * device_cu_count(), 256) * 256;
 }
 static size_t attn_split_bytes(int64_t queries, int64_t ns, int64_t ng) {
     return ns > 1 ? attn_count_bytes() + (size_t)(queries * ns * (2 + 3 * ng)) * sizeof(float) : 0;
 }
 
+// Queries of one sequence per workgroup of rq_kv_attn_kernel: 4 or 2 while the
+// workgroups still have two tiles for each wave of the device (head dim 128,
+// 256 sequences of 4096 positions: 2 queries 165 -> 117 us, 4 queries 320 ->
+// 187; 64 sequences of 534 positions, 2 queries of head dim 80: 18 us apart,
+// 20 together). Two workgroups per CU for a group, by splitting further, were
+// slower (448 sequences of 1790 positions, 4 queries: 209 us against 174).
+static int attn_group(int64_t bh, int64_t nq, int64_t T, int64_t ng) {
+    int group = 1;
+    if (ng <= 64)
+        while (group < kMaxGroup && group < nq &&
+               bh * ceil_div(nq, 2 * group) * T >= 2 * kAttnWaves * (int64_t)device_cu_count())
+            group *= 2;
+    return group;
+}
+
 static size_t attn_workspace_bytes(int64_t bh, int64_t nq, int64_t seq, int64_t dim) {
     const int64_t ng = ceil_div(dim, 3), T = ceil_div(seq, kTile);
-    const int64_t wgs = bh * nq * (ng > 64 ? ceil_div(ng, kWideRange) : 1);
+    const int64_t wgs = bh * ceil_div(nq, attn_group(bh, nq, T, ng)) * (ng > 64 ? ceil_div(ng, kWideRange) : 1);
     int64_t ns, tps;
     attn_splits(wgs, T, ng > 64, ns, tps);
     return attn_split_bytes(bh * nq, ns, ng);
@@ -691,10 +754,11 @@ extern "C" int rnn_rotorquant_kv_attention_ws(const float *q, int64_t bh, int64_
                 "%s: pages must be 16-byte aligned", name);
     RNN_REQUIRE(bh * nq <= 0x7fffffffLL, "%s: too many queries", name);
     const int64_t ng = ceil_div(dim, 3), T = ceil_div(seq, kTile);
-    const unsigned grid = (unsigned)(bh * nq);
+    const int group = attn_group(bh, nq, T, ng);
+    const unsigned grid = (unsigned)(bh * ceil_div(nq, group));
     const int64_t nranges = ng > 64 ? ceil_div(ng, kWideRange) : 1;
     int64_t ns, tps;
-    attn_splits(bh * nq * nranges, T, ng > 64, ns, tps);
+    attn_splits(grid * nranges, T, ng > 64, ns, tps);
     hipStream_t st = as_stream(stream);
     // ns > 1: the splits' states go to the workspace (or stream-ordered
     // scratch, its counts zeroed); the last split of each query (and range)
@@ -723,14 +787,20 @@ extern "C" int rnn_rotorquant_kv_attention_ws(const float *q, int64_t bh, int64_
                                  (size_t)wide_lds, st>>>(q, k_codes, k_scales, v_codes, v_scales,
                                                          k_rotors, v_rotors, nq, seq, dim, ng, T,
                                                          tps, scale, out, part, cnt);
-    } else if (ng <= 44) {
-        rq_kv_attn_kernel<11, 6><<<dim3(grid, (unsigned)ns), kAttnWaves * 64, 0, st>>>(
-            q, k_codes, k_scales, v_codes, v_scales, k_rotors, v_rotors, nq, seq, dim, ng, T, tps,
-            scale, out, part, cnt);
     } else {
-        rq_kv_attn_kernel<16, 8><<<dim3(grid, (unsigned)ns), kAttnWaves * 64, 0, st>>>(
-            q, k_codes, k_scales, v_codes, v_scales, k_rotors, v_rotors, nq, seq, dim, ng, T, tps,
-            scale, out, part, cnt);
+        auto go = [&](auto kernel) {
+            kernel<<<dim3(grid, (unsigned)ns), kAttnWaves * 64, 0, st>>>(
+                q, k_codes, k_scales, v_codes, v_scales, k_rotors, v_rotors, nq, seq, dim, ng, T, tps,
+                scale, out, part, cnt);
+        };
+        if (ng <= 44)
+            group == 1   ? go(rq_kv_attn_kernel<11, 6, 1>)
+            : group == 2 ? go(rq_kv_attn_kernel<11, 6, 2>)
+                         : go(rq_kv_attn_kernel<11, 6, 4>);
+        else
+            group == 1   ? go(rq_kv_attn_kernel<16, 8, 1>)
+            : group == 2 ? go(rq_kv_attn_kernel<16, 8, 2>)
+                         : go(rq_kv_attn_kernel<16, 8, 4>);
     }
     int rc = check_launch(name);
     if (ws && ws != workspace) {

@@ -185,3 +185,37 @@ def test_kv_attention_workspace_shared_between_shapes(dev, hip):
         for args, fresh in runs:
             out = torch.full_like(fresh, float("nan"))
             assert torch.equal(hip.rotorquant_kv_attention(*args, out=out), fresh)
+
+
+@pytest.mark.parametrize("bh,nq,seq,dim", [(3, 2, 70, 64), (2, 3, 130, 128), (1, 4, 1, 96),
+                                           (40, 5, 700, 128), (90, 4, 600, 64), (300, 2, 100, 128),
+                                           (5, 7, 1500, 190), (2, 4, 0, 128)])
+def test_kv_attention_query_groups(dev, hip, bh, nq, seq, dim):
+    """Several queries of a sequence share a workgroup (2 and 4, the last
+    group partly filled), with and without the sequence split (more counts
+    than workgroups): within the bound of float64 attention, and equal to each
+    query alone within twice it; repeated on the same workspace bit for bit."""
+    import torch
+    rng = np.random.default_rng(bh + nq + seq)
+    ng = (dim + 2) // 3
+    krot, vrot = W.rotors(ng, seed=41), W.rotors(ng, seed=42)
+    q = rng.standard_normal((bh, nq, dim)).astype(np.float32)
+    scale = float(1.0 / np.sqrt(dim))
+    if seq == 0:
+        z16, z32 = torch.zeros(8, dtype=torch.int16, device=dev), torch.zeros(8, device=dev)
+        out = hip.rotorquant_kv_attention(to_dev(q, dev), (z16, z32), (z16, z32), to_dev(krot, dev),
+                                          to_dev(vrot, dev), 0, scale)
+        assert torch.equal(out, torch.zeros_like(out))
+        return
+    kp, k = make_cache(hip, dev, W.activations(bh * seq, dim, seed=seq), krot, 4, bh, seq,
+                       hip.RQ_PAGE_K)
+    vp, v = make_cache(hip, dev, W.activations(bh * seq, dim, seed=seq + 1), vrot, 4, bh, seq,
+                       hip.RQ_PAGE_V)
+    args = (kp, vp, to_dev(krot, dev), to_dev(vrot, dev), seq, scale)
+    out = hip.rotorquant_kv_attention(to_dev(q, dev), *args)
+    exact, lim = attn64(q, k, v, scale), bound(q, k, v, scale)
+    assert np.all(np.abs(out.cpu().numpy() - exact) <= lim)
+    one = torch.cat([hip.rotorquant_kv_attention(to_dev(q[:, i:i + 1], dev), *args)
+                     for i in range(nq)], 1)
+    assert np.all(np.abs((out - one).cpu().numpy()) <= 2 * lim)
+    assert torch.equal(out, hip.rotorquant_kv_attention(to_dev(q, dev), *args))
