@@ -219,3 +219,35 @@ def test_kv_attention_query_groups(dev, hip, bh, nq, seq, dim):
                      for i in range(nq)], 1)
     assert np.all(np.abs((out - one).cpu().numpy()) <= 2 * lim)
     assert torch.equal(out, hip.rotorquant_kv_attention(to_dev(q, dev), *args))
+
+
+@pytest.mark.parametrize("bh,seq,dim", [(1, 1, 3), (3, 65, 5), (2, 64, 64), (5, 200, 80), (3, 130, 96),
+                                        (2, 1000, 128), (4, 63, 128), (2, 129, 130), (1, 700, 256),
+                                        (2, 70, 298), (1, 5, 1)])
+def test_kv_pack_tiles_match_the_scalar_kernel(dev, hip, bh, seq, dim):
+    """The tile kernel (16-byte aligned codes) against the one-thread-per-word
+    kernel, which codes one byte past an aligned address still take: every
+    element of both kinds of page, nothing written past them."""
+    import torch
+    ng = (dim + 2) // 3
+    g = torch.Generator(device=dev).manual_seed(bh + seq + dim)
+    n = bh * seq
+    buf = torch.randint(-7, 8, (n * 3 * ng + 16,), generator=g, device=dev, dtype=torch.int8)
+    scales = torch.rand((n, ng), generator=g, device=dev)
+    odd = buf[1:1 + n * 3 * ng].view(n, 3 * ng)
+    even = odd.clone()
+    nc, ns = hip.rotorquant_kv_page_elems(bh, seq, dim)
+    for kind in (hip.RQ_PAGE_K, hip.RQ_PAGE_V):
+        pages = []
+        for codes in (even, odd):
+            pc = torch.full((nc + 8,), 77, dtype=torch.int16, device=dev)
+            ps = torch.full((ns + 8,), 77.0, device=dev)
+            import ctypes
+            P = ctypes.c_void_p
+            rc = hip.load().rnn_rotorquant_kv_pack(
+                P(codes.data_ptr()), P(scales.data_ptr()), bh, seq, dim, 4, kind, P(pc.data_ptr()),
+                P(ps.data_ptr()), P(torch.cuda.current_stream().cuda_stream))
+            assert rc == hip.RNN_OK
+            pages.append((pc, ps))
+        assert torch.equal(pages[0][0], pages[1][0]) and torch.equal(pages[0][1], pages[1][1])
+        assert bool((pages[0][0][nc:] == 77).all()) and bool((pages[0][1][ns:] == 77).all())
