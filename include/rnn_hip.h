@@ -126,6 +126,15 @@ int rnn_w8a8_linear(const int8_t *aq, const float *sa, const int8_t *wq,
                     int64_t n, unsigned flags, float *y, int32_t *acc_out,
                     void *stream);
 
+/* The W8A8 layer from f32 activations (src/int8.rs:134-172 with the per-row
+ * rule): rnn_quant_rows_i8 of x [m, k] into `scratch`, then rnn_w8a8_linear
+ * (same flags, same bits as the two calls). scratch: 16-byte aligned, at least
+ * m*k rounded up to 16, plus 4*m bytes, any contents. */
+int rnn_w8a8_forward(const float *x, int64_t m, int64_t k, const int8_t *wq,
+                     const float *sw, const float *bias, int64_t n,
+                     unsigned flags, float *y, void *scratch,
+                     size_t scratch_bytes, void *stream);
+
 /* Int8Model::forward in one launch: a chain of nlayers W8A8 layers over x
  * [m, dims[0]] (the 784-256-128-10 MLP of the benchmark configurations).
  * Layer l: the running activation's rows are quantized per row
@@ -189,6 +198,14 @@ int rnn_ternary_gemm(const int8_t *aq, const float *sa, const uint32_t *packed,
                      const float *sw, const float *bias, int64_t m, int64_t k,
                      int64_t n, unsigned flags, float *y, int32_t *acc_out,
                      void *stream);
+
+/* The int8 ternary layer from f32 activations (src/ternary.rs:239-279 on int8
+ * codes): rnn_quant_rows_i8 of x [m, k] into `scratch` (sized as for
+ * rnn_w8a8_forward), then rnn_ternary_gemm. */
+int rnn_ternary_forward(const float *x, int64_t m, int64_t k,
+                        const uint32_t *packed, const float *sw,
+                        const float *bias, int64_t n, unsigned flags, float *y,
+                        void *scratch, size_t scratch_bytes, void *stream);
 
 /* The packed codes of a ternary weight [rows, cols] (TernaryTensor::packed,
  * cols % 16 == 0 so that rows are whole words) rearranged for the GEMM: within

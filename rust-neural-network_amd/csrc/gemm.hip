@@ -2249,6 +2249,44 @@ extern "C" int rnn_ternary_gemm(const int8_t *aq, const float *sa, const uint32_
     return launch_tiled<128, 128, 64, 64, true>(aq, packed, m, n, k, epi, st, name);
 }
 
+// Scratch of the two forwards below: the codes of x, then its row scales.
+static int forward_quantize(const float *x, int64_t m, int64_t k, void *scratch, size_t scratch_bytes,
+                            void *stream, const char *name, int8_t **aq, float **sa) {
+    const size_t codes = ((size_t)m * (size_t)k + 15) / 16 * 16;
+    RNN_REQUIRE(scratch && ((uintptr_t)scratch & 15) == 0 && scratch_bytes >= codes + 4 * (size_t)m,
+                "%s: scratch of %zu bytes (or misaligned), %zu needed", name, scratch_bytes,
+                codes + 4 * (size_t)m);
+    *aq = static_cast<int8_t *>(scratch);
+    *sa = reinterpret_cast<float *>(*aq + codes);
+    return rnn_quant_rows_i8(x, m, k, *aq, *sa, stream);
+}
+
+extern "C" int rnn_w8a8_forward(const float *x, int64_t m, int64_t k, const int8_t *wq, const float *sw,
+                                const float *bias, int64_t n, unsigned flags, float *y, void *scratch,
+                                size_t scratch_bytes, void *stream) {
+    RNN_ENTRY();
+    const char *name = "rnn_w8a8_forward";
+    RNN_REQUIRE(m >= 0 && k >= 0 && n >= 0, "%s: negative size", name);
+    if (m == 0 || n == 0) return RNN_OK;
+    int8_t *aq;
+    float *sa;
+    RNN_TRY(forward_quantize(x, m, k, scratch, scratch_bytes, stream, name, &aq, &sa));
+    return rnn_w8a8_linear(aq, sa, wq, sw, bias, m, k, n, flags, y, nullptr, stream);
+}
+
+extern "C" int rnn_ternary_forward(const float *x, int64_t m, int64_t k, const uint32_t *packed,
+                                   const float *sw, const float *bias, int64_t n, unsigned flags,
+                                   float *y, void *scratch, size_t scratch_bytes, void *stream) {
+    RNN_ENTRY();
+    const char *name = "rnn_ternary_forward";
+    RNN_REQUIRE(m >= 0 && k >= 0 && n >= 0, "%s: negative size", name);
+    if (m == 0 || n == 0) return RNN_OK;
+    int8_t *aq;
+    float *sa;
+    RNN_TRY(forward_quantize(x, m, k, scratch, scratch_bytes, stream, name, &aq, &sa));
+    return rnn_ternary_gemm(aq, sa, packed, sw, bias, m, k, n, flags, y, nullptr, stream);
+}
+
 // ------------------------------------------------------- ternary MFMA layout
 // One thread per 32-bit word: the 16 two-bit codes are moved to the MFMA
 // layout (ternary_word_to_mfma_layout). Rows stay word-aligned (K % 16 == 0),

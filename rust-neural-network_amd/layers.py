@@ -188,10 +188,8 @@ class Int8Linear(Module):
 
     def forward_w8a8(self, x, relu=False):
         """y = (Σ q(x)·W_q · sa[m]) · sw[n] + b[n], ReLU fused when asked."""
-        aq, sa = H.quant_rows_i8(x)
-        y, _ = H.w8a8_linear(aq, sa, self.int8_weight.data, self.int8_weight.scales, self.bias,
-                             relu=relu)
-        return y
+        return H.w8a8_forward(x, self.int8_weight.data, self.int8_weight.scales, self.bias,
+                              relu=relu)
 
 
 class Int8Model(Module):
@@ -310,7 +308,6 @@ class TernaryLinear(Module):
         16 == 0 the codes are rearranged once (rnn_ternary_prepack) into the
         layout the GEMM decodes with byte permutes; the reference-layout
         `packed` field is kept as the source of truth."""
-        aq, sa = H.quant_rows_i8(x)
         tw = self.ternary_weight
         if self.in_features % 16 == 0:
             # the prepacked copy follows `ternary_weight.packed`: another
@@ -322,12 +319,9 @@ class TernaryLinear(Module):
                 self._mfma_packed = H.ternary_prepack(tw.packed, self.out_features,
                                                       self.in_features)
                 self._mfma_src = (weakref.ref(tw.packed), tw.packed._version)
-            y, _ = H.ternary_gemm(aq, sa, self._mfma_packed, tw.scales, self.out_features,
-                                  self.bias, relu=relu, mfma_layout=True)
-        else:
-            y, _ = H.ternary_gemm(aq, sa, tw.packed, tw.scales, self.out_features, self.bias,
-                                  relu=relu)
-        return y
+            return H.ternary_forward(x, self._mfma_packed, tw.scales, self.out_features,
+                                     self.bias, relu=relu, mfma_layout=True)
+        return H.ternary_forward(x, tw.packed, tw.scales, self.out_features, self.bias, relu=relu)
 
 
 class TernaryModel(Module):
@@ -464,9 +458,9 @@ class QuantizedLinear(Module):
         """QuantizedLinear::forward (src/quantize.rs:744-754). The layer keeps
         one workspace for the GEMV, so a forward allocates nothing but its
         output (forwards of one layer are ordered on the current stream)."""
-        import torch
         w = self.weight
         if self._workspace is None:
+            import torch
             self._workspace = torch.zeros(H.qt_linear_workspace_size(self.in_features,
                                                                      self.out_features),
                                           dtype=torch.uint8, device=w.data.device)

@@ -11,6 +11,8 @@ import ctypes
 import os
 import re
 
+import torch
+
 HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(HERE, "librnn_hip.so")
 HEADER = os.path.join(os.path.dirname(HERE), "include", "rnn_hip.h")
@@ -64,6 +66,9 @@ SIGNATURES = {
     "rnn_igemm": ([_P, _P, _P, _I64, _I64, _I64, _P, ctypes.c_size_t, _P], _INT),
     "rnn_igemm_noalloc": ([_P, _P, _P, _I64, _I64, _I64, _P], _INT),
     "rnn_w8a8_linear": ([_P, _P, _P, _P, _P, _I64, _I64, _I64, _UINT, _P, _P, _P], _INT),
+    "rnn_w8a8_forward": ([_P, _I64, _I64, _P, _P, _P, _I64, _UINT, _P, _P, ctypes.c_size_t, _P], _INT),
+    "rnn_ternary_forward": ([_P, _I64, _I64, _P, _P, _P, _I64, _UINT, _P, _P, ctypes.c_size_t, _P],
+                            _INT),
     "rnn_ternary_pack": ([_P, _I64, _P, _P], _INT),
     "rnn_ternary_unpack": ([_P, _I64, _P, _P], _INT),
     "rnn_ternary_quantize": ([_P, _I64, _I64, _INT, _P, _P, _P], _INT),
@@ -137,17 +142,24 @@ def _check(status: int):
 
 
 def _ptr(t):
-    return None if t is None else ctypes.c_void_p(t.data_ptr())
+    return None if t is None else t.data_ptr()
+
+
+# The current stream's handle without building a Stream object (2.8 -> 0.1 us
+# a call); torch versions without these names take the public one.
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+_raw_device = getattr(torch._C, "_cuda_getDevice", None)
 
 
 def _stream(stream):
-    import torch
-    s = stream if stream is not None else torch.cuda.current_stream()
-    return ctypes.c_void_p(s.cuda_stream)
+    if stream is not None:
+        return stream.cuda_stream
+    if _raw_stream is None or _raw_device is None:
+        return torch.cuda.current_stream().cuda_stream
+    return _raw_stream(_raw_device())
 
 
 def _dev(t, dtype, name):
-    import torch
     if t is None:
         return None
     if not t.is_cuda:
@@ -187,7 +199,6 @@ def _dims(t, nd, name):
 
 
 def _empty(shape, dtype, like):
-    import torch
     return torch.empty(shape, dtype=dtype, device=like.device)
 
 
@@ -195,18 +206,17 @@ def _scratch(nbytes, like, stream):
     """(device bytes for one call, or None; the call's stream), from torch's
     allocator in the pool of that stream: freed at the end of the call, they
     are handed out again only to work ordered behind it."""
-    import torch
-    s = _stream(stream)
     if not nbytes:
-        return None, s
+        return None, _stream(stream)
+    if stream is None:
+        return torch.empty(nbytes, dtype=torch.uint8, device=like.device), _stream(None)
     with torch.cuda.stream(stream):
-        return torch.empty(nbytes, dtype=torch.uint8, device=like.device), s
+        return torch.empty(nbytes, dtype=torch.uint8, device=like.device), stream.cuda_stream
 
 
 # ------------------------------------------------------------------ int8
 def quant_rows_i8(x, q=None, scale=None, stream=None):
     """Per-row symmetric int8 (Int8Weights::quantize rule). Returns (q, scale)."""
-    import torch
     _dev(x, torch.float32, "x")
     rows, cols = _dims(x, 2, "x")
     q = _out(q, torch.int8, rows * cols, "q") if q is not None else _empty((rows, cols), torch.int8, x)
@@ -217,7 +227,6 @@ def quant_rows_i8(x, q=None, scale=None, stream=None):
 
 
 def int8_dequantize(q, scale, stream=None):
-    import torch
     _dev(q, torch.int8, "q"), _dev(scale, torch.float32, "scale")
     rows, _ = _dims(q, 2, "q")
     _need(scale, rows, "scale")
@@ -228,7 +237,6 @@ def int8_dequantize(q, scale, stream=None):
 
 
 def int8_matmul_f32(wq, ws, x, stream=None):
-    import torch
     _dev(wq, torch.int8, "wq"), _dev(ws, torch.float32, "ws"), _dev(x, torch.float32, "x")
     out_f, in_f = _dims(wq, 2, "wq")
     _need(ws, out_f, "ws")
@@ -242,7 +250,6 @@ def int8_matmul_f32(wq, ws, x, stream=None):
 
 
 def int8_linear_forward(x, wq, ws, bias=None, stream=None):
-    import torch
     _dev(x, torch.float32, "x"), _dev(wq, torch.int8, "wq"), _dev(ws, torch.float32, "ws")
     _dev(bias, torch.float32, "bias")
     batch, in_f = _dims(x, 2, "x")
@@ -262,7 +269,6 @@ def igemm_workspace_size(m, k, n) -> int:
 
 def igemm(a_u8, b_i8, m, k, n, workspace=None, c=None, stream=None):
     """igemm contract: a u8 [m,k], b i8 [k,n] -> c i32 [m,n]."""
-    import torch
     _dev(a_u8, torch.uint8, "a"), _dev(b_i8, torch.int8, "b")
     if min(m, k, n) < 0:
         raise RnnError(RNN_ERR_INVALID_ARG, f"negative size m={m} k={k} n={n}")
@@ -282,7 +288,6 @@ IGEMM_NOALLOC_MAX_BYTES = 64 << 20  # RNN_IGEMM_NOALLOC_MAX_BYTES
 def igemm_noalloc(a_u8, b_i8, m, k, n, c, stream=None):
     """igemm into a caller-allocated c (int32 [m, n]) with the library's
     device-array workspace: no allocation anywhere in the call."""
-    import torch
     _dev(a_u8, torch.uint8, "a"), _dev(b_i8, torch.int8, "b")
     if min(m, k, n) < 0:
         raise RnnError(RNN_ERR_INVALID_ARG, f"negative size m={m} k={k} n={n}")
@@ -294,7 +299,6 @@ def igemm_noalloc(a_u8, b_i8, m, k, n, c, stream=None):
 def w8a8_linear(aq, sa, wq, sw, bias=None, relu=False, algo=ALGO_AUTO, want_y=True,
                 want_acc=False, y=None, acc=None, stream=None):
     """Returns (y f32 [m,n] or None, acc i32 [m,n] or None)."""
-    import torch
     _dev(aq, torch.int8, "aq"), _dev(wq, torch.int8, "wq")
     _dev(sa, torch.float32, "sa"), _dev(sw, torch.float32, "sw"), _dev(bias, torch.float32, "bias")
     m, k = _dims(aq, 2, "aq")
@@ -313,6 +317,24 @@ def w8a8_linear(aq, sa, wq, sw, bias=None, relu=False, algo=ALGO_AUTO, want_y=Tr
     return y, acc
 
 
+def w8a8_forward(x, wq, sw, bias=None, relu=False, stream=None):
+    """quant_rows_i8 + w8a8_linear in one call (the codes and scales of x in
+    the call's scratch): y [m, n] f32 of x [m, k] f32."""
+    _dev(x, torch.float32, "x"), _dev(wq, torch.int8, "wq"), _dev(sw, torch.float32, "sw")
+    _dev(bias, torch.float32, "bias")
+    m, k = _dims(x, 2, "x")
+    n, wk = _dims(wq, 2, "wq")
+    if wk != k:
+        raise RnnError(RNN_ERR_INVALID_ARG, f"x has k={k}, wq has k={wk}")
+    _need(sw, n, "sw"), _need(bias, n, "bias")
+    y = _empty((m, n), torch.float32, x)
+    need = (m * k + 15) // 16 * 16 + 4 * m
+    ws, s = _scratch(need, x, stream)
+    _check(load().rnn_w8a8_forward(_ptr(x), m, k, _ptr(wq), _ptr(sw), _ptr(bias), n,
+                                   FLAG_RELU if relu else 0, _ptr(y), _ptr(ws), need, s))
+    return y
+
+
 def w8a8_mlp(x, layers, relu=True, y=None, stream=None):
     """A chain of W8A8 layers in one launch (rnn_w8a8_mlp): `layers` is a list
     of (wq [n, k] int8, sw [n] f32, bias [n] f32 or None); x [m, k0] f32.
@@ -320,7 +342,6 @@ def w8a8_mlp(x, layers, relu=True, y=None, stream=None):
     layers when `relu`. Raises RnnError (RNN_ERR_UNSUPPORTED) for chains the
     single launch does not take (more than 4 layers, widths over 1024,
     in-features not a multiple of 16)."""
-    import torch
     _dev(x, torch.float32, "x")
     m, k0 = _dims(x, 2, "x")
     nl = len(layers)
@@ -339,16 +360,13 @@ def w8a8_mlp(x, layers, relu=True, y=None, stream=None):
     w = (ctypes.c_void_p * nl)(*[l[0].data_ptr() for l in layers])
     s_ = (ctypes.c_void_p * nl)(*[l[1].data_ptr() for l in layers])
     b_ = (ctypes.c_void_p * nl)(*[0 if l[2] is None else l[2].data_ptr() for l in layers])
-    _check(load().rnn_w8a8_mlp(_ptr(x), m, nl, ctypes.cast(d, ctypes.c_void_p),
-                               ctypes.cast(w, ctypes.c_void_p), ctypes.cast(s_, ctypes.c_void_p),
-                               ctypes.cast(b_, ctypes.c_void_p), int(bool(relu)), _ptr(y),
+    _check(load().rnn_w8a8_mlp(_ptr(x), m, nl, d, w, s_, b_, int(bool(relu)), _ptr(y),
                                _stream(stream)))
     return y
 
 
 # ------------------------------------------------------------------ ternary
 def ternary_pack(t, stream=None):
-    import torch
     _dev(t, torch.int8, "t")
     count = t.numel()
     packed = _empty(((count + 15) // 16,), torch.int32, t)
@@ -357,7 +375,6 @@ def ternary_pack(t, stream=None):
 
 
 def ternary_unpack(packed, count, stream=None):
-    import torch
     _dev(packed, torch.int32, "packed")
     _need(packed, (count + 15) // 16, "packed", at_least=True)
     t = _empty((count,), torch.int8, packed)
@@ -367,7 +384,6 @@ def ternary_unpack(packed, count, stream=None):
 
 def ternary_quantize(w, mode=TERNARY_ROWS, stream=None):
     """Returns (packed int32 words [ceil(numel/16)], scales f32 [rows])."""
-    import torch
     _dev(w, torch.float32, "w")
     rows, cols = _dims(w, 2, "w")
     packed = _empty(((rows * cols + 15) // 16,), torch.int32, w)
@@ -378,7 +394,6 @@ def ternary_quantize(w, mode=TERNARY_ROWS, stream=None):
 
 
 def ternary_dequantize(packed, numel, scales, cols, stream=None):
-    import torch
     _dev(packed, torch.int32, "packed"), _dev(scales, torch.float32, "scales")
     _need(packed, (numel + 15) // 16, "packed", at_least=True)
     w = _empty((numel,), torch.float32, packed)
@@ -388,7 +403,6 @@ def ternary_dequantize(packed, numel, scales, cols, stream=None):
 
 
 def ternary_linear_forward(x, packed, scales, out_f, bias=None, stream=None):
-    import torch
     _dev(x, torch.float32, "x"), _dev(packed, torch.int32, "packed")
     _dev(scales, torch.float32, "scales"), _dev(bias, torch.float32, "bias")
     batch, in_f = _dims(x, 2, "x")
@@ -403,7 +417,6 @@ def ternary_linear_forward(x, packed, scales, out_f, bias=None, stream=None):
 def ternary_prepack(packed, rows, cols, stream=None):
     """The MFMA code layout of a ternary weight [rows, cols] (cols % 16 == 0):
     same size, read by ternary_gemm(..., mfma_layout=True)."""
-    import torch
     _dev(packed, torch.int32, "packed")
     _need(packed, rows * cols // 16, "packed", at_least=True)
     out = _empty((rows * cols // 16,), torch.int32, packed)
@@ -413,7 +426,6 @@ def ternary_prepack(packed, rows, cols, stream=None):
 
 def ternary_gemm(aq, sa, packed, sw, n, bias=None, relu=False, want_y=True, want_acc=False,
                  y=None, stream=None, algo=ALGO_AUTO, mfma_layout=False):
-    import torch
     _dev(aq, torch.int8, "aq"), _dev(packed, torch.int32, "packed")
     _dev(sa, torch.float32, "sa"), _dev(sw, torch.float32, "sw"), _dev(bias, torch.float32, "bias")
     m, k = _dims(aq, 2, "aq")
@@ -429,9 +441,24 @@ def ternary_gemm(aq, sa, packed, sw, n, bias=None, relu=False, want_y=True, want
     return y, acc
 
 
+def ternary_forward(x, packed, sw, n, bias=None, relu=False, mfma_layout=False, stream=None):
+    """quant_rows_i8 + ternary_gemm in one call, as w8a8_forward."""
+    _dev(x, torch.float32, "x"), _dev(packed, torch.int32, "packed")
+    _dev(sw, torch.float32, "sw"), _dev(bias, torch.float32, "bias")
+    m, k = _dims(x, 2, "x")
+    _need(packed, (n * k + 15) // 16, "packed", at_least=True)
+    _need(sw, n, "sw"), _need(bias, n, "bias")
+    y = _empty((m, n), torch.float32, x)
+    need = (m * k + 15) // 16 * 16 + 4 * m
+    ws, s = _scratch(need, x, stream)
+    flags = (FLAG_RELU if relu else 0) | (FLAG_TERNARY_MFMA_LAYOUT if mfma_layout else 0)
+    _check(load().rnn_ternary_forward(_ptr(x), m, k, _ptr(packed), _ptr(sw), _ptr(bias), n, flags,
+                                      _ptr(y), _ptr(ws), need, s))
+    return y
+
+
 # ------------------------------------------------------------------ RotorQuant
 def rotation_matrices(rotors, stream=None):
-    import torch
     _dev(rotors, torch.float32, "rotors")
     n = rotors.shape[0] if rotors.dim() > 0 else 0
     _need(rotors, 4 * n, "rotors")
@@ -442,7 +469,6 @@ def rotation_matrices(rotors, stream=None):
 
 def rotorquant_quantize(x, rotors, bits, want_y=True, want_codes=False, y=None, stream=None):
     """Returns (y or None, codes int8 [rows,padded] or None, scales [rows,groups] or None)."""
-    import torch
     _dev(x, torch.float32, "x"), _dev(rotors, torch.float32, "rotors")
     dim = x.shape[-1]
     rows = x.numel() // dim if dim else 0
@@ -459,7 +485,6 @@ def rotorquant_quantize(x, rotors, bits, want_y=True, want_codes=False, y=None, 
 
 
 def rotorquant_dequantize(codes, scales, dim, rotors, stream=None):
-    import torch
     _dev(codes, torch.int8, "codes"), _dev(scales, torch.float32, "scales")
     _dev(rotors, torch.float32, "rotors")
     ng = (dim + 2) // 3
@@ -478,7 +503,6 @@ def sgemm(transa, transb, m, n, k, alpha, a, lda, b, ldb, beta, c, ldc, stream=N
     C = alpha*op(A)*op(B) + beta*C on device storage `a`, `b`, `c` (f32
     tensors holding the row-major matrices with row strides lda/ldb/ldc).
     `transa`/`transb` are NO_TRANS or TRANS. C is updated in place."""
-    import torch
     for t, nm in ((a, "a"), (b, "b"), (c, "c")):
         _dev(t, torch.float32, nm)
 
@@ -496,7 +520,6 @@ def sgemm(transa, transb, m, n, k, alpha, a, lda, b, ldb, beta, c, ldc, stream=N
 
 def matmul(a, b, stream=None):
     """blas::matmul (src/blas.rs:780-799): C = A.B for contiguous [m,k] @ [k,n]."""
-    import torch
     _dev(a, torch.float32, "a"), _dev(b, torch.float32, "b")
     m, k = _dims(a, 2, "a")
     kb, n = _dims(b, 2, "b")
@@ -509,7 +532,6 @@ def matmul(a, b, stream=None):
 def relu(x, out=None, stream=None):
     """Tensor::relu (src/tensor.rs:2025-2032): x.max(0.0) elementwise (NaN -> 0).
     `out` may be x itself."""
-    import torch
     _dev(x, torch.float32, "x")
     out = _out(out, torch.float32, x.numel(), "out") if out is not None else torch.empty_like(x)
     _check(load().rnn_relu(_ptr(x), x.numel(), _ptr(out), _stream(stream)))
@@ -519,7 +541,6 @@ def relu(x, out=None, stream=None):
 def bias_act(y, bias=None, relu=False, stream=None):
     """The fused bias add + activation of Tensor::linear_layer
     (src/tensor.rs:771-786), in place on y [rows, cols]."""
-    import torch
     _dev(y, torch.float32, "y"), _dev(bias, torch.float32, "bias")
     rows, cols = _dims(y, 2, "y")
     _need(bias, cols, "bias")
@@ -530,7 +551,6 @@ def bias_act(y, bias=None, relu=False, stream=None):
 def linear_layer(x, w, bias=None, relu=False, out=None, stream=None):
     """Tensor::linear_layer (src/tensor.rs:747-800): act(x [batch, in] . W^T +
     b) with W stored [out, in]; bias may be None (Linear without bias)."""
-    import torch
     _dev(x, torch.float32, "x"), _dev(w, torch.float32, "w"), _dev(bias, torch.float32, "bias")
     batch, in_f = _dims(x, 2, "x")
     out_f, w_in = _dims(w, 2, "w")
@@ -571,7 +591,6 @@ def qt_layout(fmt, n, group_size):
 def qt_quantize(fmt, x, group_size, stream=None):
     """QuantizedTensor::quantize of the flat data of device tensor x. Returns
     (data uint8 [bytes], scales f32 [groups], stored group_size)."""
-    import torch
     _dev(x, torch.float32, "x")
     n = x.numel()
     nb, ns, g = qt_layout(fmt, n, group_size)
@@ -584,7 +603,6 @@ def qt_quantize(fmt, x, group_size, stream=None):
 
 def qt_dequantize(fmt, data, scales, group, n, stream=None):
     """QuantizedTensor::dequantize (src/quantize.rs:252-269): flat f32 [n]."""
-    import torch
     _dev(data, torch.uint8, "data"), _dev(scales, torch.float32, "scales")
     out = _empty((n,), torch.float32, data)
     _check(load().rnn_qt_dequantize(fmt, _ptr(data), data.numel(), _ptr(scales), scales.numel(),
@@ -602,7 +620,6 @@ def qt_linear_forward(fmt, x, data, scales, group, out_f, bias=None, algo=ALGO_A
     `workspace`: a zeroed device byte tensor of at least
     qt_linear_workspace_size(in, out) bytes for the bf16 MFMA GEMV's scratch
     (else the call allocates); calls leave it reusable."""
-    import torch
     _dev(x, torch.float32, "x"), _dev(data, torch.uint8, "data")
     _dev(scales, torch.float32, "scales"), _dev(bias, torch.float32, "bias")
     _dev(workspace, torch.uint8, "workspace")
@@ -638,7 +655,6 @@ def rotorquant_kv_pack(codes, scales, bh, seq, dim, bits, kind, stream=None):
     """Codes/scales of rotorquant_quantize (rows = bh*seq) -> a KV-cache page
     of the given kind (RQ_PAGE_K or RQ_PAGE_V): (u16 codes as int16, f32
     scales), both flat."""
-    import torch
     _dev(codes, torch.int8, "codes"), _dev(scales, torch.float32, "scales")
     ng = (dim + 2) // 3
     _need(codes, bh * seq * 3 * ng, "codes"), _need(scales, bh * seq * ng, "scales")
@@ -660,8 +676,8 @@ _attn_ws = {}
 
 
 def _attn_workspace(dev, nbytes):
-    import torch
-    key = (dev, torch.cuda.current_stream(dev).cuda_stream)
+    key = (dev, _raw_stream(dev.index) if _raw_stream and dev.index is not None
+           else torch.cuda.current_stream(dev).cuda_stream)
     ws = _attn_ws.get(key)
     if ws is None or ws.numel() < nbytes:
         ws = torch.zeros(nbytes, dtype=torch.uint8, device=dev)
@@ -678,7 +694,6 @@ def rotorquant_kv_attention(q, k_page, v_page, k_rotors, v_rotors, seq, scale, o
     the sequence split's states (calls leave it reusable); on the current
     stream a cached one is used when none is given, on another stream the
     call allocates."""
-    import torch
     _dev(q, torch.float32, "q")
     for t, nm in ((k_page[0], "k codes"), (v_page[0], "v codes")):
         _dev(t, torch.int16, nm)
