@@ -42,7 +42,7 @@ enum rnn_status {
 
 /* flags for the GEMM entry points */
 #define RNN_FLAG_RELU 0x1u          /* y = max(y, 0) after bias (src/tensor.rs:2025-2032) */
-#define RNN_ALGO_AUTO 0x00u         /* GEMV for m <= 16, else LDS-DMA tiles (k % 128 == 0, n % 4 == 0) or register-staged tiles */
+#define RNN_ALGO_AUTO 0x00u         /* GEMV for m <= 16, else the tile shape with the smallest estimated time (k % 16 == 0), or the byte-assembling tiles */
 #define RNN_ALGO_TILED 0x10u        /* force the register-staged 128x128 MFMA GEMM */
 #define RNN_ALGO_GEMV 0x20u         /* force the skinny GEMV (m <= 16; rnn_qt_linear_forward: per 16-row slice for any m) */
 #define RNN_ALGO_TILED_DMA 0x30u    /* force the LDS-DMA pipelined big-tile GEMM (k % 128 == 0, n % 4 == 0) */

@@ -171,6 +171,23 @@ def test_igemm_small_unaligned_operands(dev, hip):
     assert np.array_equal(got, O.igemm_scalar(a, b, m, k, n))
 
 
+@pytest.mark.parametrize("m,k,n", [(33, 257, 95), (5, 31, 31), (64, 288, 33), (2, 32, 32),
+                                   (31, 1023, 65), (70, 33, 161)])
+def test_igemm_unaligned_wide_loads(dev, hip, m, k, n):
+    """The small igemm at sizes and addresses that are not multiples of 16: 32-byte
+    pieces wholly inside a row are loaded at any address, pieces that cross the
+    row's end byte by byte; the operands end where their storage ends."""
+    import torch
+    a, b = lcg_case(m, k, n)
+    exp = O.igemm_scalar(a, b, m, k, n)
+    for off in (0, 1, 7):
+        ab = torch.zeros(m * k + off, dtype=torch.uint8, device=dev)
+        bb = torch.zeros(k * n + off, dtype=torch.int8, device=dev)
+        ab[off:], bb[off:] = to_dev(a.ravel(), dev), to_dev(b.ravel(), dev)
+        got = hip.igemm(ab[off:].view(m, k), bb[off:].view(k, n), m, k, n)
+        assert np.array_equal(host(got), exp)
+
+
 def test_igemm_wrapping(dev, hip):
     m, k, n = 2, 70016, 3
     a = np.full((m, k), 255, np.uint8)
