@@ -711,8 +711,9 @@ static void attn_splits(int64_t wgs, int64_t T, bool wide, int group, int64_t &n
     ns = 1;
     if (wgs < want && T >= 2 * kAttnWaves)
         // (a group's workgroups have a CU each, so a few past the CUs would take
-        // a second round: rounded down. 192 queries of 2478 positions, head dim
-        // 64, in pairs: 2 splits 30 us against 60 for 3)
+        // a second round: rounded down. 96 sequences of 2478 positions, 2 queries
+        // of head dim 64: 39 us with 2 splits, 60 with 3, both with the kernel
+        // of head dim 132; 30 with its own)
         ns = std::min<int64_t>({group > 1 ? want / wgs : ceil_div(want, wgs), T / kAttnWaves, kMaxSplits});
     tps = ceil_div(T, ns);
     ns = T > 0 ? ceil_div(T, tps) : 1;  // no empty split
@@ -737,8 +738,8 @@ static size_t attn_split_bytes(int64_t queries, int64_t ns, int64_t ng) {
 // Queries of one sequence per workgroup of rq_kv_attn_kernel: 4 or 2 while the
 // workgroups still have two tiles for each wave of the device (head dim 128,
 // 256 sequences of 4096 positions: 2 queries 165 -> 117 us, 4 queries 320 ->
-// 187; 64 sequences of 534 positions, 2 queries of head dim 80: 18 us apart,
-// 20 together). Two workgroups per CU for a group, by splitting further, were
+// 187; 64 sequences of 534 positions, 2 queries of head dim 80, with the kernel
+// of dim 132: 18 us apart, 20 together). Two workgroups per CU for a group, by splitting further, were
 // slower (448 sequences of 1790 positions, 4 queries: 209 us against 174).
 static int attn_group(int64_t bh, int64_t nq, int64_t T, int64_t ng) {
     int group = 1;
@@ -898,14 +899,19 @@ extern "C" int rnn_rotorquant_kv_attention_ws(const float *q, int64_t bh, int64_
                 q, k_codes, k_scales, v_codes, v_scales, k_rotors, v_rotors, nq, seq, dim, ng, T, tps,
                 scale, out, part, cnt);
         };
-        if (ng <= 44)
-            group == 1   ? go(rq_kv_attn_kernel<11, 6, 1>)
-            : group == 2 ? go(rq_kv_attn_kernel<11, 6, 2>)
-                         : go(rq_kv_attn_kernel<11, 6, 4>);
-        else
-            group == 1   ? go(rq_kv_attn_kernel<16, 8, 1>)
-            : group == 2 ? go(rq_kv_attn_kernel<16, 8, 2>)
-                         : go(rq_kv_attn_kernel<16, 8, 4>);
+#define RNN_ATTN(NG4, NG8)                                   \
+    (group == 1   ? go(rq_kv_attn_kernel<NG4, NG8, 1>)      \
+     : group == 2 ? go(rq_kv_attn_kernel<NG4, NG8, 2>)      \
+                  : go(rq_kv_attn_kernel<NG4, NG8, 4>))
+        // Groups a kernel scores: head dims up to 72, 96, 132 and 192. The arrays
+        // of a smaller kernel leave registers for more loads in flight (300
+        // sequences of 1000 positions, 2 queries of head dim 64: 59 us with the
+        // 132 kernel, 30 with its own; 256 of 2048, 4 queries of 96: 93 and 78).
+        if (ng <= 24) RNN_ATTN(6, 3);
+        else if (ng <= 32) RNN_ATTN(8, 4);
+        else if (ng <= 44) RNN_ATTN(11, 6);
+        else RNN_ATTN(16, 8);
+#undef RNN_ATTN
     }
     int rc = check_launch(name);
     if (ws && ws != workspace) {

@@ -221,6 +221,35 @@ def test_kv_attention_query_groups(dev, hip, bh, nq, seq, dim):
     assert torch.equal(out, hip.rotorquant_kv_attention(to_dev(q, dev), *args))
 
 
+@pytest.mark.parametrize("nq,seq", [(3, 650), (3, 1290), (2, 1300)])
+@pytest.mark.parametrize("dim", [5, 72, 73, 96, 97, 132, 133, 192])
+def test_kv_attention_full_query_groups(dev, hip, nq, seq, dim):
+    """104 sequences (4 distinct ones) give the device's waves enough tiles for
+    groups of 2 (the second one partly filled), 4 (partly filled, split over
+    the sequence) and 2 (split), at the head dims where the kernels' sizes
+    change: within the bound of float64 attention, a second call equal."""
+    bh, few = 104, 4
+    rng = np.random.default_rng(seq + dim)
+    ng = (dim + 2) // 3
+    krot, vrot = W.rotors(ng, seed=43), W.rotors(ng, seed=44)
+    q = rng.standard_normal((bh, nq, dim)).astype(np.float32)
+    scale = float(1.0 / np.sqrt(dim))
+    pages, recon = [], []
+    for rot, kind, seed in ((krot, hip.RQ_PAGE_K, 1), (vrot, hip.RQ_PAGE_V, 2)):
+        x = W.activations(few * seq, dim, seed=seed)
+        _, codes, scales = hip.rotorquant_quantize(to_dev(x, dev), to_dev(rot, dev), 4,
+                                                   want_y=False, want_codes=True)
+        r = O.rotorquant_dequantize(codes.cpu().numpy(), scales.cpu().numpy(), dim, rot)
+        recon.append(np.tile(r.reshape(few, seq, dim), (bh // few, 1, 1)))
+        pages.append(hip.rotorquant_kv_pack(codes.repeat(bh // few, 1), scales.repeat(bh // few, 1),
+                                            bh, seq, dim, 4, kind))
+    args = (to_dev(q, dev), *pages, to_dev(krot, dev), to_dev(vrot, dev), seq, scale)
+    out = hip.rotorquant_kv_attention(*args)
+    k, v = recon
+    assert np.all(np.abs(out.cpu().numpy() - attn64(q, k, v, scale)) <= bound(q, k, v, scale))
+    assert (out == hip.rotorquant_kv_attention(*args)).all()
+
+
 @pytest.mark.parametrize("bh,seq,dim", [(1, 1, 3), (3, 65, 5), (2, 64, 64), (5, 200, 80), (3, 130, 96),
                                         (2, 1000, 128), (4, 63, 128), (2, 129, 130), (1, 700, 256),
                                         (2, 70, 298), (1, 5, 1)])
