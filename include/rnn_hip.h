@@ -119,7 +119,10 @@ int rnn_igemm_noalloc(const uint8_t *a, const int8_t *b, int32_t *c, int64_t m,
  * Int8Weights layout, src/int8.rs:14-17). Any k and any operand alignment
  * (the igemm contract, src/int8.rs:288-296): k % 16 != 0 or unaligned operands
  * take a tiled kernel that assembles its chunks from byte loads (the forced
- * GEMV and LDS-DMA algos need k % 16 == 0 and 16-byte alignment).
+ * GEMV and LDS-DMA algos need k % 16 == 0 and 16-byte alignment). AUTO takes
+ * the GEMV for m <= 16 and otherwise the tile shape whose estimated time is
+ * the smallest (256 x 224 tiles for large outputs, small tiles with K split
+ * over a workgroup's waves where the output has few tiles).
  * bias, y and acc_out may each be NULL (not both y and acc_out). */
 int rnn_w8a8_linear(const int8_t *aq, const float *sa, const int8_t *wq,
                     const float *sw, const float *bias, int64_t m, int64_t k,
@@ -189,9 +192,10 @@ int rnn_ternary_linear_forward(const float *x, int64_t batch, int64_t in_f,
  * the 2-bit codes inside the kernel, acc = sum_k aq[m,k]*t[n,k], epilogue as
  * rnn_w8a8_linear with sw[n].
  * flags: RNN_FLAG_RELU, RNN_FLAG_TERNARY_MFMA_LAYOUT when `packed` comes
- * from rnn_ternary_prepack (k % 16 == 0), and an algo (AUTO: the LDS-DMA
- * kernel when k % 128 == 0, n % 4 == 0 and buffers are 16-byte aligned, else
- * TILED; TILED or TILED_DMA force one). Any k is accepted in the reference
+ * from rnn_ternary_prepack (k % 16 == 0), and an algo (AUTO: of the LDS-DMA
+ * kernels that take the shape -- 64 x 128 tiles for k % 128 == 0 and n % 4 ==
+ * 0, the small tiles for k % 16 == 0, buffers 16-byte aligned -- the one with
+ * the smaller estimated time, else TILED; TILED or TILED_DMA force one). Any k is accepted in the reference
  * layout: rows that start mid-word (k % 16 != 0) or unaligned activations take
  * a tiled kernel that gathers codes from arbitrary bit offsets. */
 int rnn_ternary_gemm(const int8_t *aq, const float *sa, const uint32_t *packed,
@@ -378,7 +382,9 @@ int rnn_qt_dequantize(int format, const uint8_t *data, int64_t data_bytes,
  * route: up to m = 512 when the slices take the bf16 MFMA GEMV with 4-bit
  * codes, 192 with 8-bit codes or bf16 weights, 96 for the f32 MFMA GEMV, 32
  * for the VALU GEMV; otherwise
- * dequantize into stream-ordered scratch and run rnn_sgemm. RNN_ALGO_GEMV,
+ * dequantize into stream-ordered scratch and run rnn_sgemm
+ * (rnn_qt_linear_forward_scratch has a faster route above 48 rows).
+ * RNN_ALGO_GEMV,
  * _GEMV_MFMA and _GEMV_BF16 force their GEMV (per 16-row slice for any m;
  * error if it does not fit), RNN_ALGO_TILED the dequantize route. f32 sums in
  * the kernel's own order: within the rnn_sgemm rounding bound of the

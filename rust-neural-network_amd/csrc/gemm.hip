@@ -2,7 +2,8 @@
 //
 //   acc[m,n] = sum_k A[m,k] * B[n,k]     A [M,K] int8, B [N,K] int8 (both
 //                                        K-contiguous: the Int8Weights layout)
-// Entry points: rnn_w8a8_linear (W8A8 with fused dequant epilogue), rnn_igemm
+// Entry points: rnn_w8a8_linear (W8A8 with fused dequant epilogue; the small
+// tiles are in gemm_mid.hpp), rnn_w8a8_forward (with the quantizer), rnn_igemm
 // (the reference's u8 x i8 [K,N] contract via a pack step + zero-point
 // correction) and rnn_ternary_gemm (B = 2-bit codes decoded in the tile loader).
 #include <algorithm>
@@ -2003,7 +2004,8 @@ static bool dma_ok(const int8_t *A, const int8_t *B, int64_t N, int64_t K, const
            al(epi.acc_out) && al(epi.sw) && al(epi.bias) && al(epi.colsum);
 }
 
-// Block-tile choice for the LDS-DMA kernel: for M > 128, 256x224 tiles with
+// Block-tile choice for the LDS-DMA kernels (RNN_ALGO_TILED_DMA; AUTO compares
+// with the small tiles, launch_w8a8_auto): for M > 128, 256x224 tiles with
 // 8 waves (2 per SIMD, 64x112 int32 accumulators each, so one wave's barrier
 // and DMA waits overlap the other's MFMAs; 2048x14336 is 512 tiles = two full
 // rounds on 256 CUs, one block per CU for the 128 KiB LDS ring), else 128x128

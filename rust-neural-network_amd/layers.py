@@ -440,8 +440,9 @@ class QuantizedTensor:
 
 class QuantizedLinear(Module):
     """src/quantize.rs:718-754: a quantized weight `[out, in]` and optional
-    f32 bias. `forward` decodes the weight inside the GEMV (or dequantizes
-    once and runs the f32 GEMM for many rows)."""
+    f32 bias. `forward` decodes the weight inside the GEMV, or for many
+    rows inside a tiled product on the matrix cores (formats and groups that
+    does not take are dequantized for the f32 product)."""
 
     def __init__(self, weight, bias, in_features, out_features):
         self.weight, self.bias = weight, bias

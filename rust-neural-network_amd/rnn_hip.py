@@ -619,7 +619,8 @@ def qt_linear_forward(fmt, x, data, scales, group, out_f, bias=None, algo=ALGO_A
     """QuantizedLinear::forward (src/quantize.rs:744-754): x [m, in] -> y [m, out].
     `workspace`: a zeroed device byte tensor of at least
     qt_linear_workspace_size(in, out) bytes for the bf16 MFMA GEMV's scratch
-    (else the call allocates); calls leave it reusable."""
+    (else the call allocates); calls leave it reusable. Above 16 rows the
+    call's other scratch comes from torch's allocator."""
     _dev(x, torch.float32, "x"), _dev(data, torch.uint8, "data")
     _dev(scales, torch.float32, "scales"), _dev(bias, torch.float32, "bias")
     _dev(workspace, torch.uint8, "workspace")
