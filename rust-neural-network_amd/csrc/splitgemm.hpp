@@ -156,6 +156,11 @@ struct SplitWF32 {
     static __device__ __forceinline__ float at(const void *w, int64_t ldw, int64_t n, int64_t k, float) {
         return *reinterpret_cast<const float *>(static_cast<const uint8_t *>(w) + n * ldw + 4 * k);
     }
+    static __device__ __forceinline__ sg_f4 at4(const void *w, int64_t ldw, int64_t n, int64_t k, float) {
+        const float *p = reinterpret_cast<const float *>(static_cast<const uint8_t *>(w) + n * ldw) + k;
+        if constexpr (ALIGNED) return *reinterpret_cast<const sg_f4 *>(p);
+        return sg_f4{p[0], p[1], p[2], p[3]};
+    }
 };
 
 enum { SPLIT_I4, SPLIT_I8, SPLIT_BF16, SPLIT_E2M1 };
@@ -215,11 +220,36 @@ struct SplitWQ {
             return __uint_as_float((uint32_t)reinterpret_cast<const uint16_t *>(row)[k] << 16);
         else if constexpr (FMT == SPLIT_I8)
             return (float)(int8_t)row[k] * s;
-        const uint32_t nib = (row[k / 2] >> (4 * (k & 1))) & 15u;
-        if constexpr (FMT == SPLIT_I4) return (float)((int)(nib << 28) >> 28) * s;
+        return nibble(row[k / 2] >> (4 * (k & 1))) * s;
+    }
+    // elements k .. k + 3 (k % 4 == 0)
+    static __device__ __forceinline__ sg_f4 at4(const void *w, int64_t ldw, int64_t n, int64_t k, float s) {
+        const uint8_t *row = static_cast<const uint8_t *>(w) + n * ldw;
+        sg_f4 v;
+        if constexpr (FMT == SPLIT_BF16) {
+            uint32_t d[2];
+            __builtin_memcpy(d, row + 2 * k, 8);
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+                v[e] = __uint_as_float(e & 1 ? d[e / 2] & 0xFFFF0000u : d[e / 2] << 16);
+        } else if constexpr (FMT == SPLIT_I8) {
+            uint32_t d;
+            __builtin_memcpy(&d, row + k, 4);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) v[e] = (float)(int8_t)(d >> (8 * e)) * s;
+        } else {
+            uint16_t d;
+            __builtin_memcpy(&d, row + k / 2, 2);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) v[e] = nibble((uint32_t)d >> (4 * e)) * s;
+        }
+        return v;
+    }
+    static __device__ __forceinline__ float nibble(uint32_t nib) {  // of the low 4 bits
+        if constexpr (FMT == SPLIT_I4) return (float)((int)(nib << 28) >> 28);
         const float mag = nib & 4 ? (nib & 2 ? (nib & 1 ? 6.0f : 4.0f) : (nib & 1 ? 3.0f : 2.0f))
                                   : 0.5f * (float)(nib & 3);
-        return (nib & 8 ? -mag : mag) * s;
+        return nib & 8 ? -mag : mag;
     }
 };
 
@@ -494,24 +524,65 @@ void split_gemm_kernel(SplitArgs a) {
 #pragma unroll
     for (int v = 0; v < 8; ++v) any |= flags[v];
     if (any) {
+        // Each wave its own fragments, TM + TN operand loads for TN TM of them.
+        // Per 16 k, lane group fq takes k + 4 fq .. + 3 of both operands (one
+        // 16-byte load where x is aligned); a pass is 32 k. Bound by the loads'
+        // latency and lines. With every tile computed again, 2000 x 4096 x 4096
+        // f32 takes 1.1 ms and Q8_0 300 x 4096 x 11008 1.08 (one fragment at a
+        // time in steps of 4 k: 7.4 and 5.4 ms; without such values 0.38, 0.14).
         const int64_t k0 = 32 * (int64_t)s0, k1 = std::min<int64_t>(a.K, 32 * (int64_t)(s0 + steps));
+        const bool vec = (a.ldx & 3) == 0 && ((uintptr_t)a.x & 15) == 0;
 #pragma unroll
-        for (int f = 0; f < C::F; ++f) {
-            if (WK > 1 && f % WK != kg) continue;
-            const int64_t m = std::min(mw + 16 * (f % TM) + fr, a.M - 1);
-            const int64_t n = std::min(nw + 16 * (f / TM) + fr, a.N - 1);
-            sg_f4 v = {0.f, 0.f, 0.f, 0.f};
+        for (auto &row : acc)
+#pragma unroll
+            for (auto &v : row) v = sg_f4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll 1
-            for (int64_t k = k0 + fq; k - fq < k1; k += 4) {
-                const int64_t kc = std::min(k, k1 - 1);
-                const float s = W::SCALED ? a.scales[n * a.sc_n / a.sc_d +
-                                                     (a.sc_k ? (uint32_t)(kc / 32) / a.sc_k : 0)]
-                                          : 1.0f;
-                float xv = a.x[m * a.ldx + kc], wv = W::at(a.w, a.ldw, n, kc, s);
-                if (k >= k1) xv = 0.0f, wv = 0.0f;
-                v = __builtin_amdgcn_mfma_f32_16x16x4f32(xv, wv, v, 0, 0, 0);
+        for (int64_t kb = k0; kb < k1; kb += 32) {
+            const bool whole = kb + 32 <= k1;
+            sg_f4 xv[2][TM], wv[2][TN];
+#pragma unroll
+            for (int u = 0; u < TM; ++u) {
+                const float *const xr = a.x + std::min(mw + 16 * u + fr, a.M - 1) * a.ldx;
+#pragma unroll
+                for (int h = 0; h < 2; ++h) {
+                    const int64_t k = kb + 16 * h + 4 * fq;
+                    if (whole && vec) {
+                        xv[h][u] = *reinterpret_cast<const sg_f4 *>(xr + k);
+                    } else {
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) xv[h][u][e] = k + e < k1 ? xr[k + e] : 0.0f;
+                    }
+                }
             }
-            acc[f / TM][f % TM] = v;
+#pragma unroll
+            for (int t = 0; t < TN; ++t) {
+                const int64_t n = std::min(nw + 16 * t + fr, a.N - 1);
+                float s = 1.0f;
+                if constexpr (W::SCALED)
+                    s = a.scales[n * a.sc_n / a.sc_d + (a.sc_k ? (uint32_t)(kb / 32) / a.sc_k : 0)];
+#pragma unroll
+                for (int h = 0; h < 2; ++h) {
+                    const int64_t k = kb + 16 * h + 4 * fq;
+                    if (whole) {
+                        wv[h][t] = W::at4(a.w, a.ldw, n, k, s);
+                    } else {
+#pragma unroll
+                        for (int e = 0; e < 4; ++e)
+                            wv[h][t][e] = k + e < k1 ? W::at(a.w, a.ldw, n, k + e, s) : 0.0f;
+                    }
+                }
+            }
+#pragma unroll
+            for (int h = 0; h < 2; ++h)
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+#pragma unroll
+                    for (int t = 0; t < TN; ++t)
+#pragma unroll
+                        for (int u = 0; u < TM; ++u)
+                            if (WK == 1 || (t * TM + u) % WK == kg)
+                                acc[t][u] = __builtin_amdgcn_mfma_f32_16x16x4f32(
+                                    xv[h][u][e], wv[h][t][e], acc[t][u], 0, 0, 0);
         }
     }
     // lane: rows mw + 16 u + 4 fq + e, column nw + 16 t + fr

@@ -99,6 +99,21 @@ def test_linear_layer_split_values_the_parts_do_not_hold(dev, hip):
     assert torch.equal(clean, hip.linear_layer(x, w))
 
 
+@pytest.mark.parametrize("k", [481, 497, 510, 543])
+def test_linear_layer_split_computed_again_k_remainders(dev, hip, k):
+    """Tiles computed again in f32 where K ends within a pass of 32: the bound
+    of an f32 sum in any order, (k + 4) U sum |x||w|."""
+    import torch
+    m, n = 140, 300
+    x, w, b = data(m, k, n, k)
+    x[::16, 5] = 2.0 ** -120
+    w[::32, k - 1] = 2.0 ** -125
+    assert hip.load().rnn_linear_layer_workspace_size(w.data_ptr(), m, k, n) > 0
+    ref = x.double() @ w.double().t() + b.double()
+    lim = (k + 4) * U * (x.double().abs() @ w.double().abs().t() + b.double().abs())
+    assert bool(((hip.linear_layer(x, w, b).double() - ref).abs() <= lim).all())
+
+
 def test_linear_layer_split_capture_and_streams(dev, hip):
     """Replays of a captured call, and a call on another stream, give the
     eager bits (the parts live in the call's own scratch)."""
